@@ -169,6 +169,13 @@ constexpr int kWideRecGroups = 1 + HD / 32 * 16 / 4;
 // 512 over 1.8-3.7k contexts): the first, second and third workgroup of each CU finished at 197,
 // 207 and 218 us (medians), i.e. progressed at relative rates 1.10 : 1.05 : 1.
 __device__ __forceinline__ int share_weight(int s) { return s < 2 ? 22 - s : 20; }
+// Gangs that share W steps: at most as many as leave each at least one step, the smallest weight's
+// included. A gang without steps would be counted among the pieces of a cut tile and never arrive.
+// (The grid follows the page table's width, W the requests' lengths, which may be far shorter.)
+__device__ __forceinline__ int share_gangs(int W, int gangs) {
+  const int most = (int)((int64_t)W * share_weight(2) / share_weight(0));
+  return most < 1 ? 1 : (gangs < most ? gangs : most);
+}
 
 template <int HD>
 constexpr int kWideRecFloats = kWideWaves * kWideRecGroups<HD> * kWave * 4;
@@ -331,10 +338,11 @@ void prefill_wide_kernel(const AttnArgs a) {
     }
     __syncthreads();
     W = HP * __builtin_amdgcn_readfirstlane(sS[a.B]);
+    NG = share_gangs(W, NG);
     if (threadIdx.x <= NG) sLo[threadIdx.x] = (int)((int64_t)W * sCw[threadIdx.x] / sCw[NG]);
     __syncthreads();
-    lo = __builtin_amdgcn_readfirstlane(sLo[gang]);
-    hi = __builtin_amdgcn_readfirstlane(sLo[gang + 1]);
+    lo = gang < NG ? __builtin_amdgcn_readfirstlane(sLo[gang]) : 0;  // (no share past the last gang)
+    hi = gang < NG ? __builtin_amdgcn_readfirstlane(sLo[gang + 1]) : 0;
     // First pair of the share: request pb = the last with HP * S[pb] <= lo (S[0] = 0).
     int lb = 0, ub = a.B - 1;
     while (lb < ub) {
@@ -807,10 +815,11 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(co
     }
     __syncthreads();
     W = HP * __builtin_amdgcn_readfirstlane(sS[a.B]);
+    NG = share_gangs(W, NG);
     if (threadIdx.x <= NG) sLo[threadIdx.x] = (int)((int64_t)W * sCw[threadIdx.x] / sCw[NG]);
     __syncthreads();
-    lo = __builtin_amdgcn_readfirstlane(sLo[gang]);
-    hi = __builtin_amdgcn_readfirstlane(sLo[gang + 1]);
+    lo = gang < NG ? __builtin_amdgcn_readfirstlane(sLo[gang]) : 0;  // (no share past the last gang)
+    hi = gang < NG ? __builtin_amdgcn_readfirstlane(sLo[gang + 1]) : 0;
     int lb = 0, ub = a.B - 1;
     while (lb < ub) {
       const int mid = (lb + ub + 1) / 2;
