@@ -721,31 +721,59 @@ void prefill_wide_kernel(const AttnArgs a) {
   }  // pieces
 }
 
-// fp32 KV: the same workgroup layout, LDS staging and online softmax, on v_mfma_f32_32x32x2_f32
-// (fp32 products, like the reference's fp32 path):
-//   S^T = K Q^T      MFMA s (s < HD/2) contracts head_dim slot G2 = index G2*HD/2 + s: lane
-//                    (G2, c) gives K[key c][index] (A, from LDS) and q[query c][index] (B, held
-//                    in registers for the whole walk);
-//   O^T += V^T P^T   MFMA (j, r) contracts key slot G2 = key 8j + 4*G2 + r, the key whose score
-//                    lane (G2, c) holds in its register 4j + r: A = V[that key][c*DU + d] (output
-//                    tile d, row c) and B = its softmax weight, exactly as held.
-// Per 32-key step a wavefront issues HD MFMAs of 32x32x2 (HD/2 for QK^T, HD/2 for PV), so the
-// per-step costs are small next to the matrix work.
+// fp32 KV: the bf16 kernel's workgroup layout, operand layouts and online softmax, with every fp32
+// operand as the sum of three bf16 parts (split_bf16x3: 8 + 8 + 8 significant bits, exact to
+// 2^-26 of the value) and every fp32 product as the six partial products whose parts' indices add
+// up to at most 4, on v_mfma_f32_32x32x16_bf16 with fp32 accumulation. The dropped partial products
+// are below 2^-25 of the product, i.e. below fp32's own rounding of it.
+//   bound: the matrix cores. The fp32 MFMA (32x32x2) runs at 1/16 of the bf16 rate, so six bf16
+//   products take 6/16 of its time; a 32-key step at head_dim 128 is 96 bf16 MFMAs of 32 cycles
+//   against 128 fp32 ones of 64. K and V are split once per workgroup (not once per wavefront) on
+//   their way into LDS: K planes 0-2, V planes 3-5, each 32 unpadded key rows of bf16, swizzled as
+//   in the bf16 kernel. The next step's fp32 values wait in registers meanwhile, so one LDS stage
+//   (48 KB at head_dim 128) is enough and two workgroups share a compute unit.
+//   error: the scores' leading products are accumulated apart from the rest, in 8 (not 64) rounded
+//   additions, an output in 12 (not 16) per 32 keys. 4 x 32 heads x 128, 512-token chunks over
+//   1-4k, N(0, 1): 8e-7 of the output's norm against float64; fp32 MFMA 1e-6.
+//   measured (MI355X, the same shape, chunk append included): 948 -> 605 us; at 4k contexts 185
+//   TFLOP/s, 55% MFMA and 31% VALU busy at a clock that the load pulls down to 1.75 GHz (all-zero
+//   operands run a quarter faster), i.e. 1110 TFLOP/s of bf16 products, where a large plain bf16
+//   matrix product reaches 1200-1600 on the same kind of data.
+// A value of 2^60 or more (an infinity among them) has no such split whose products stay finite: a
+// wavefront whose q or whose workgroup's K or V held one walks its steps a second time, with
+// v_mfma_f32_32x32x2_f32 on operands read straight from memory (slow; fp32 products as they are).
+// NaN needs no care: its parts are NaN.
+constexpr float kSplitMax = 1152921504606846976.f;  // 2^60
+
+// Two fp32 values as packed bf16 triples: x = w1 + w2 + w3, each part the nearest bf16 of the rest.
+__device__ __forceinline__ void split_bf16x3(float lo, float hi, uint32_t& w1, uint32_t& w2, uint32_t& w3) {
+  w1 = pack_bf16x2(lo, hi);
+  lo -= bf16_lo(w1);
+  hi -= bf16_hi(w1);
+  w2 = pack_bf16x2(lo, hi);
+  lo -= bf16_lo(w2);
+  hi -= bf16_hi(w2);
+  w3 = pack_bf16x2(lo, hi);
+}
+
 template <typename IO, int HD, bool BAL>
-__global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(kWideWaves * kWave) __attribute__((amdgpu_waves_per_eu(2)))
+void prefill_wide_f32_kernel(const AttnArgs a) {
   constexpr int NW = kWideWaves;
   constexpr int KS = 32;                 // keys per step (two 16-token blocks)
   constexpr int NBS = 2;
   constexpr int QH = HD / 2;             // head_dim values per lane in the QK^T operands
+  constexpr int NQ = HD / 16;            // contraction slices of 16 per score
   constexpr int DU = HD / 32;            // output tiles of 32 head_dim rows
-  constexpr int RS = HD + 4;             // LDS row stride in floats (16-byte pad)
-  constexpr int RPC = HD / 4;            // 16-byte chunks per key row
-  constexpr int CPT = KS * RPC / (NW * kWave);
-  static_assert(CPT >= 1 && KS * RPC == CPT * NW * kWave, "tile split");
+  constexpr int CPR = HD / 8;            // 8-value chunks (16 bytes of a plane) per key row
+  constexpr int RPB = 128 / HD;          // key rows of a plane per 256 bytes (one pass over the banks)
+  constexpr int PLANE = KS * HD;         // elements per plane
+  constexpr int CPT = KS * CPR / (NW * kWave);  // chunks per thread per K (or V) tile
+  static_assert(CPT >= 1 && KS * CPR == CPT * NW * kWave, "tile split");
   static_assert(!BAL || HD == 128 || HD == 64, "balanced launch shape");
 
-  __shared__ __attribute__((aligned(16))) float sk[2][KS * RS];
-  __shared__ __attribute__((aligned(16))) float sv[2][KS * RS];
+  __shared__ __attribute__((aligned(16))) uint16_t sbuf[6 * PLANE];
+  __shared__ int sm_bad;  // number of the last piece that held a K or V value past kSplitMax
 
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -782,8 +810,8 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(co
     return lg;
   };
   if constexpr (!BAL) {
-    static_assert(sizeof(sk) >= (kOrderMax + 1) * sizeof(int), "order scratch");
-    if (!wide_lpt_unit(a, ntiles, reinterpret_cast<int*>(&sk[0][0]), bh, qt)) wide_unit(blockIdx.x, a.B * a.H, ntiles, bh, qt);
+    static_assert(sizeof(sbuf) >= (kOrderMax + 1) * sizeof(int), "order scratch");
+    if (!wide_lpt_unit(a, ntiles, reinterpret_cast<int*>(sbuf), bh, qt)) wide_unit(blockIdx.x, a.B * a.H, ntiles, bh, qt);
   } else {
     k = blockIdx.x % kXcds;
     const int jx = blockIdx.x / kXcds;
@@ -831,6 +859,9 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(co
     P = __builtin_amdgcn_readfirstlane(sS[pb + 1]) - Sb;
     hh = (int)((lo - HP * Sb) / P);
   }
+  int piece = 0;
+  if (threadIdx.x == 0) sm_bad = 0;
+  __syncthreads();
   for (bool first = true;; first = false) {
   int b, h, s_hi = 0x7fffffff;
   int s_lo = 0, np = 1, g0 = 0, rec_slot = 0;
@@ -878,15 +909,29 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(co
     wsteps = wsteps < nsteps ? wsteps : nsteps;
   }
 
-  // B operand of S^T = K Q^T: q[i][G2*QH + s], pre-scaled into the log2 domain.
-  float qf[QH];
-  {
-    const IO* qp = static_cast<const IO*>(a.q) + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh +
-                   (int64_t)(i < a.T ? i : 0) * a.q_st + G2 * QH;
-    const float qs = i < a.T ? a.scale_log2 : 0.f;
+  // B operand of S^T = K Q^T: q[i][G2*QH + 8s + e] for slice s, pre-scaled into the log2 domain, in
+  // three parts.
+  const IO* qp = static_cast<const IO*>(a.q) + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh +
+                 (int64_t)(i < a.T ? i : 0) * a.q_st + G2 * QH;
+  const float qs = i < a.T ? a.scale_log2 : 0.f;
+  bf16x8 qb[3][NQ];
+  float qmax = 0.f;
 #pragma unroll
-    for (int s = 0; s < QH; ++s) qf[s] = Elem<IO>::load(qp + s) * qs;
+  for (int s = 0; s < NQ; ++s) {
+    u32x4 w1, w2, w3;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = Elem<IO>::load(qp + 8 * s + 2 * e) * qs, y = Elem<IO>::load(qp + 8 * s + 2 * e + 1) * qs;
+      qmax = fmaxf(fmaxf(qmax, fabsf(x)), fabsf(y));
+      uint32_t p1, p2, p3;
+      split_bf16x3(x, y, p1, p2, p3);
+      w1[e] = p1; w2[e] = p2; w3[e] = p3;
+    }
+    qb[0][s] = __builtin_bit_cast(bf16x8, w1);
+    qb[1][s] = __builtin_bit_cast(bf16x8, w2);
+    qb[2][s] = __builtin_bit_cast(bf16x8, w3);
   }
+  const bool q_bad = __builtin_amdgcn_ballot_w64(qmax >= kSplitMax) != 0;
 
   f32x16 oacc[DU];
 #pragma unroll
@@ -901,68 +946,83 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(co
   // Page-table entries are int32: one unsigned 32-bit compare checks 0 <= e < num_blocks.
   const uint32_t nblk = a.num_blocks < 0x7fffffff ? (uint32_t)a.num_blocks : 0x7fffffffu;
   auto ok_blk = [&](int e) { return (uint32_t)e < nblk; };
+  auto blk_off = [&](int e) {  // (masked in the softmax when invalid)
+    return ((int64_t)(ok_blk(e) ? e : 0) * a.H + h) * (16 * HD);
+  };
+  // Chunk swizzles of the bf16 kernel's K and V tiles.
+  auto kswz = [](int r) { return (r / RPB) & (CPR - 1); };
+  auto vswz = [](int r) { return (4 * ((r / RPB) & 3)) & (CPR - 1); };
 
-  u32x4 kr[CPT], vr[CPT];
+  f32x4 kr[CPT][2], vr[CPT][2];
   auto gload = [&](int st, int (&ent)[NBS]) {
 #pragma unroll
     for (int j = 0; j < NBS; ++j) ent[j] = NBS * st + j < nb ? pt[NBS * st + j] : -1;
 #pragma unroll
     for (int n = 0; n < CPT; ++n) {
       const int q = threadIdx.x + n * NW * kWave;
-      const int kk = q / RPC;
-      const int col = (q - kk * RPC) * 4;
-      const int e = ent[kk >> 4];
-      const int blk = ok_blk(e) ? e : 0;  // masked in the softmax when invalid
-      const int64_t off = (((int64_t)blk * a.H + h) * 16 + (kk & 15)) * HD + col;
-      kr[n] = *reinterpret_cast<const u32x4*>(kpool + off);
-      vr[n] = *reinterpret_cast<const u32x4*>(vpool + off);
+      const int kk = q / CPR, p = q % CPR;
+      const int64_t off = blk_off(kk < 16 ? ent[0] : ent[1]) + (kk & 15) * HD + 8 * p;
+      const f32x4* kp = reinterpret_cast<const f32x4*>(kpool + off);
+      const f32x4* vp = reinterpret_cast<const f32x4*>(vpool + off);
+      kr[n][0] = kp[0]; kr[n][1] = kp[1];
+      vr[n][0] = vp[0]; vr[n][1] = vp[1];
     }
   };
-  auto lstore = [&](int buf) {
+  ++piece;
+  auto lstore = [&]() {
+    float mx = 0.f;
+    auto put = [&](const f32x4 (&x)[2], uint16_t* dst) {
+      u32x4 w1, w2, w3;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float lo = x[e >> 1][2 * (e & 1)], hi = x[e >> 1][2 * (e & 1) + 1];
+        mx = fmaxf(fmaxf(mx, fabsf(lo)), fabsf(hi));
+        uint32_t p1, p2, p3;
+        split_bf16x3(lo, hi, p1, p2, p3);
+        w1[e] = p1; w2[e] = p2; w3[e] = p3;
+      }
+      *reinterpret_cast<u32x4*>(dst) = w1;
+      *reinterpret_cast<u32x4*>(dst + PLANE) = w2;
+      *reinterpret_cast<u32x4*>(dst + 2 * PLANE) = w3;
+    };
 #pragma unroll
     for (int n = 0; n < CPT; ++n) {
       const int q = threadIdx.x + n * NW * kWave;
-      const int kk = q / RPC;
-      const int col = (q - kk * RPC) * 4;
-      *reinterpret_cast<u32x4*>(&sk[buf][kk * RS + col]) = kr[n];
-      *reinterpret_cast<u32x4*>(&sv[buf][kk * RS + col]) = vr[n];
+      const int kk = q / CPR, p = q % CPR;
+      put(kr[n], sbuf + kk * HD + 8 * (p ^ kswz(kk)));
+      put(vr[n], sbuf + 3 * PLANE + kk * HD + 8 * (p ^ vswz(kk)));
     }
+    if (mx >= kSplitMax) sm_bad = piece;
   };
 
-  auto compute = [&](int buf, int st, const int (&ent)[NBS]) {
-    // ---- S^T = K Q^T ------------------------------------------------------------------------
-    f32x16 sacc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) sacc[e] = 0.f;
-    const float* krow = &sk[buf][c * RS + G2 * QH];
-#pragma unroll
-    for (int s = 0; s < QH; s += 4) {
-      const f32x4 kv = *reinterpret_cast<const f32x4*>(krow + s);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[e], qf[s + e], sacc, 0, 0, 0);
-    }
-    // ---- online softmax (keys 8j + 4*G2 + r of this step) --------------------------------------
+  // Per-lane LDS offsets of the operand reads (as in the bf16 kernel).
+  const int kx = kswz(c);
+  const int vr4 = (c & 15) >> 2;
+  const int vx = vswz(4 * G2 + vr4);
+  auto v_off = [&](int d) {
+    const int hd = 32 * d + 16 * (c >> 4) + 4 * (c & 3);
+    return (4 * G2 + vr4) * HD + 8 * ((hd >> 3) ^ vx) + (hd & 4);
+  };
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+  f32x16 sacc;
+  // Online softmax over the scores of step st (keys 8j + 4*G2 + r), in place.
+  auto softmax = [&](int st, const int (&ent)[NBS]) {
     const bool ok0 = ok_blk(ent[0]), ok1 = ok_blk(ent[1]);
     const bool full = ok0 && ok1 && __builtin_amdgcn_ballot_w64(n_c < (st + 1) * KS) == 0;
-    float p[16];
-    float mloc = -INFINITY;
-    if (full) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        p[e] = sacc[e];
-        mloc = fmaxf(mloc, p[e]);
-      }
-    } else {
+    if (!full) {
       const int t0 = st * KS + 4 * G2;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int t = t0 + 8 * j + r;
-          p[4 * j + r] = ((j < 2 ? ok0 : ok1) && t < n_c) ? sacc[4 * j + r] : -INFINITY;
-          mloc = fmaxf(mloc, p[4 * j + r]);
+          sacc[4 * j + r] = ((j < 2 ? ok0 : ok1) && t < n_c) ? sacc[4 * j + r] : -INFINITY;
         }
     }
+    float mloc = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, sacc[e]);
     mloc = max_xor32(mloc);
     const bool grow = mloc > m + kRescaleSlack;
     if (__builtin_amdgcn_ballot_w64(grow) != 0) {
@@ -976,32 +1036,64 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(co
     float ps = 0.f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      p[e] = fast_exp2(p[e] - m);
-      ps += p[e];
+      sacc[e] = fast_exp2(sacc[e] - m);
+      ps += sacc[e];
     }
     l += sum_xor32(ps);
-    // ---- O^T += V^T P^T: four keys (one row group j) at a time ----------------------------------
-    // At raised wavefront priority, as in the bf16 kernel.
+  };
+  // S^T = K Q^T: the leading parts' products in sacc, the others apart.
+  auto scores = [&]() {
+    f32x16 rest;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sacc[e] = rest[e] = 0.f;
+#pragma unroll
+    for (int s = 0; s < NQ; ++s) {
+      const uint16_t* kp = sbuf + c * HD + 8 * ((G2 * (CPR / 2) + s) ^ kx);
+      const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(kp);
+      const bf16x8 k2 = *reinterpret_cast<const bf16x8*>(kp + PLANE);
+      const bf16x8 k3 = *reinterpret_cast<const bf16x8*>(kp + 2 * PLANE);
+      rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k3, qb[0][s], rest, 0, 0, 0);
+      sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, qb[0][s], sacc, 0, 0, 0);
+      rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, qb[2][s], rest, 0, 0, 0);
+      rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k2, qb[1][s], rest, 0, 0, 0);
+      rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k2, qb[0][s], rest, 0, 0, 0);
+      rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, qb[1][s], rest, 0, 0, 0);
+    }
+    sacc += rest;
+  };
+  // O^T += V^T P^T: slice mm contracts keys 16mm + 8jj + 4*G2 + r at slot (G2, 4jj + r), the lane's
+  // registers 8mm + 4jj + r; small partial products first. At raised wavefront priority, as in the
+  // bf16 kernel.
+  auto weigh = [&]() {
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float vv[4][DU];
+    for (int mm = 0; mm < 2; ++mm) {
+      u32x4 w1, w2, w3;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float* vp = &sv[buf][(8 * j + 4 * G2 + r) * RS + c * DU];
-        if constexpr (DU == 4) {
-          const f32x4 x = *reinterpret_cast<const f32x4*>(vp);
-          vv[r][0] = x[0]; vv[r][1] = x[1]; vv[r][2] = x[2]; vv[r][3] = x[3];
-        } else {
-          const u32x2 x = *reinterpret_cast<const u32x2*>(vp);
-          vv[r][0] = __uint_as_float(x[0]); vv[r][1] = __uint_as_float(x[1]);
-        }
+      for (int e = 0; e < 4; ++e) {
+        uint32_t p1, p2, p3;
+        split_bf16x3(sacc[8 * mm + 2 * e], sacc[8 * mm + 2 * e + 1], p1, p2, p3);
+        w1[e] = p1; w2[e] = p2; w3[e] = p3;
       }
+      const bf16x8 p1 = __builtin_bit_cast(bf16x8, w1), p2 = __builtin_bit_cast(bf16x8, w2),
+                   p3 = __builtin_bit_cast(bf16x8, w3);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int d = 0; d < DU; ++d)
-          oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[r][d], p[4 * j + r], oacc[d], 0, 0, 0);
+      for (int d = 0; d < DU; ++d) {
+        const uint16_t* vp = sbuf + 3 * PLANE + v_off(d) + 16 * mm * HD;
+        auto part = [&](const uint16_t* x) {
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(x));
+          const s16x4 hi =
+              __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(x + 8 * HD));
+          return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        const bf16x8 v1 = part(vp), v2 = part(vp + PLANE), v3 = part(vp + 2 * PLANE);
+        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v3, p1, oacc[d], 0, 0, 0);
+        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p3, oacc[d], 0, 0, 0);
+        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, p2, oacc[d], 0, 0, 0);
+        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, p1, oacc[d], 0, 0, 0);
+        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p2, oacc[d], 0, 0, 0);
+        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p1, oacc[d], 0, 0, 0);
+      }
     }
     __builtin_amdgcn_s_setprio(0);
   };
@@ -1009,16 +1101,58 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(co
   if (s_lo < nsteps) {
     int cur[NBS], nxt[NBS];
     gload(s_lo, cur);
-    lstore(0);
+    lstore();
     __syncthreads();
     for (int st = s_lo; st < nsteps; ++st) {
       const bool more = st + 1 < nsteps;
+      if (st < wsteps) {
+        scores();
+        softmax(st, cur);
+      }
+      // The next step's loads go out between the two products: their 32 registers are free only
+      // once the scores' operands are, and the second product covers their latency.
+      __builtin_amdgcn_sched_barrier(0);
       if (more) gload(st + 1, nxt);
-      if (st < wsteps) compute((st - s_lo) & 1, st, cur);
-      if (more) lstore((st + 1 - s_lo) & 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (st < wsteps) weigh();
+      if (!more) break;
+      __syncthreads();  // every wavefront has read this step's tiles
+      lstore();
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < NBS; ++j) cur[j] = nxt[j];
+    }
+    if (q_bad || __builtin_amdgcn_readfirstlane(sm_bad) == piece) {
+      // The second walk: fp32 products, operands from memory. Scores: MFMA slot G2 of index s is
+      // head_dim G2*QH + s. Output: slot G2 of (j, r) is key 8j + 4*G2 + r, register 4j + r.
+      m = kNegBig;
+      l = 0.f;
+#pragma unroll
+      for (int d = 0; d < DU; ++d)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[d][e] = 0.f;
+#pragma unroll 1
+      for (int st = s_lo; st < wsteps; ++st) {
+#pragma unroll
+        for (int j = 0; j < NBS; ++j) cur[j] = NBS * st + j < nb ? pt[NBS * st + j] : -1;
+        const int64_t o0 = blk_off(cur[0]), o1 = blk_off(cur[1]);
+        const float* kp = kpool + (c < 16 ? o0 : o1) + (c & 15) * HD + G2 * QH;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sacc[e] = 0.f;
+#pragma unroll 1
+        for (int s = 0; s < QH; ++s)
+          sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(kp[s], Elem<IO>::load(qp + s) * qs, sacc, 0, 0, 0);
+        softmax(st, cur);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float* vp = vpool + (j < 2 ? o0 : o1) + (8 * (j & 1) + 4 * G2 + r) * HD + c;
+#pragma unroll
+            for (int d = 0; d < DU; ++d)
+              oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vp[32 * d], sacc[4 * j + r], oacc[d], 0, 0, 0);
+          }
+      }
     }
   }
 
@@ -1093,17 +1227,16 @@ __global__ __launch_bounds__(kWideWaves * kWave) void prefill_wide_f32_kernel(co
     }
   }
 
+  // ---- write: lane holds O^T rows 8j + 4*G2 + r (head_dim 32d + row) of query column c ----------
   if (store && i < a.T) {
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  IO* op = static_cast<IO*>(a.out) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + (int64_t)i * a.o_st;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    IO* op = static_cast<IO*>(a.out) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + (int64_t)i * a.o_st;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+    for (int d = 0; d < DU; ++d)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int R = 8 * j + 4 * G2 + r;
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int d = 0; d < DU; ++d) Elem<IO>::store(op + R * DU + d, oacc[d][4 * j + r] * inv);
-    }
+        for (int r = 0; r < 4; ++r) Elem<IO>::store(op + 32 * d + 8 * j + 4 * G2 + r, oacc[d][4 * j + r] * inv);
   }
   if constexpr (!BAL) {
     break;

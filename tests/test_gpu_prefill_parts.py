@@ -1,0 +1,94 @@
+"""The fp32 wide prefill kernel forms fp32 products from three bf16 parts per operand: against float64 at
+ordinary values, and against the 16-row kernel (fp32 matrix instructions) where a part would overflow."""
+import pytest
+import torch
+
+from src.kernels.hip_paged_attention import paged_attention_prefill_hip
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(Hd, lens, T, seed, scale=1.0, dtype=torch.float32):
+    g = torch.Generator().manual_seed(seed)
+    B, H = len(lens), 8
+    pages = max(-(-n // 16) for n in lens) + 1
+    k, v = (torch.randn(B * pages, H, 16, Hd, generator=g) * scale for _ in range(2))
+    table = torch.randperm(B * pages, generator=g).view(B, pages).to(torch.int32)
+    q = torch.randn(B, H, T, Hd, generator=g).to(dtype)
+    cur = [min(n, T) for n in lens]
+    return q, k, v, table, lens, cur
+
+
+def _run(case, device, monkeypatch, kernel, balance="off"):
+    q, k, v, table, lens, cur = case
+    monkeypatch.setenv("PAGED_HIP_PREFILL_KERNEL", kernel)
+    monkeypatch.setenv("PAGED_HIP_PREFILL_BALANCE", balance)
+    return paged_attention_prefill_hip(q.to(device), k.to(device), v.to(device), table.to(device),
+                                       torch.tensor(lens, dtype=torch.int32, device=device),
+                                       torch.tensor(cur, dtype=torch.int32, device=device)).cpu()
+
+
+def _f64(case):
+    q, k, v, table, lens, cur = case
+    out = torch.zeros(q.shape, dtype=torch.float64)
+    for b, (n, c) in enumerate(zip(lens, cur)):
+        kk, vv = (p[table[b].long()].transpose(0, 1).reshape(q.shape[1], -1, q.shape[3])[:, :n].double() for p in (k, v))
+        s = q[b].double() @ kk.transpose(1, 2).contiguous() / q.shape[3] ** 0.5
+        limit = torch.clamp(n - c + 1 + torch.arange(q.shape[2]), max=n)
+        s.masked_fill_(torch.arange(n)[None, :] >= limit[:, None], float("-inf"))
+        out[b] = torch.softmax(s, -1) @ vv
+    return out
+
+
+@pytest.mark.parametrize("balance", ["off", "force"])
+@pytest.mark.parametrize("Hd", [64, 128])
+@pytest.mark.parametrize("lens,T", [([1], 1), ([33, 31, 32], 33), ([130, 700, 257], 129), ([1500], 300)], ids=str)
+def test_error_of_fp32_sums(device, monkeypatch, Hd, lens, T, balance):
+    case = _case(Hd, lens, T, Hd + T)
+    want = _f64(case)
+    got = _run(case, device, monkeypatch, "wide", balance)
+    err = float((got.double() - want).norm() / want.norm())
+    # at most 12 rounded additions per 32 keys and output, each half an ulp of the running sum at most and
+    # of either sign; 4 more for the scores, the weights and the division
+    assert err <= 2.0**-24 * (4 + (12 * max(lens) / 32) ** 0.5), err
+
+
+@pytest.mark.parametrize("balance", ["off", "force"])
+@pytest.mark.parametrize("Hd", [64, 128])
+@pytest.mark.parametrize("where", ["k", "v", "q"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), -3.4028234663852886e38, 3e38, 2.0**61])
+def test_values_without_a_finite_split(device, monkeypatch, where, value, Hd, balance):
+    lens, T = [150, 70], 140
+    case = _case(Hd, lens, T, 3)
+    q, k, v, table, _, _ = case
+    if where == "q":
+        q[0, 1, 137, 5] = value
+        q[1, 2, 3, Hd - 1] = value
+    else:
+        pool = k if where == "k" else v
+        pool[table[0, 2], 1, 3, 7] = value        # key 35 of request 0
+        pool[table[1, 4], 3, 5, Hd - 2] = value   # its last keys
+    got = _run(case, device, monkeypatch, "wide", balance)
+    ref = _run(case, device, monkeypatch, "tile")
+    # A NaN row may come out as NaN or as 0 (no positive weight sum); all else agrees, to 1e-5 (float32
+    # sums of up to 150 keys in another order) of the row's largest value.
+    bound = 1e-5 * ref.nan_to_num(0, 0, 0).abs().amax(-1, keepdim=True).clamp(min=1.0).expand_as(ref)
+    both = got.isfinite() & ref.isfinite()
+    assert bool(((got - ref).abs() <= bound)[both & (got != 0) & (ref != 0)].all())
+    clean = torch.ones_like(ref, dtype=torch.bool)  # rows that see no planted value
+    if where == "q":
+        clean[0, 1, 137] = clean[1, 2, 3] = False
+    else:
+        # (row 25 of request 0 sees keys 0-35; a masked key's weight is 0, and 0 * inf is NaN)
+        clean[0, 1, 25 if where == "k" else 0:] = clean[1, 3] = False
+    assert bool(both[clean].all())
+    if abs(value) < 1e30:  # (a larger value times a weight of up to 2^8 overflows)
+        assert bool(both.all())
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12])
+def test_scales_far_from_one(device, monkeypatch, scale):
+    q, k, v, table, lens, cur = _case(128, [300, 90], 140, 9)
+    case = (q / scale, k * scale, v * scale, table, lens, cur)
+    got, ref = _run(case, device, monkeypatch, "wide"), _run(case, device, monkeypatch, "tile")
+    assert float((got - ref).abs().max()) < 1e-5 * scale
