@@ -2,7 +2,8 @@
 
 Every `csrc/*.hip` file is compiled to an object under `_build/` and linked into
 `libpaged_hip.so` next to this file; `csrc/host/paged_host.cpp` becomes the CPython module
-`src/cache/_paged_host` (native host bookkeeping of graph steps). The library links against the HIP runtime that torch bundles
+`src/cache/_paged_host` (native host bookkeeping of graph steps) and `csrc/host/paged_call.cpp`
+`src/kernels/_paged_call` (native front of the per-layer entry points). The library links against the HIP runtime that torch bundles
 (rpath to torch/lib), so a process that imports torch and then loads the library maps a single
 HIP runtime. Usage: `python build_lib.py [--verbose]`.
 """
@@ -73,6 +74,7 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 
 HOST_SRC = CSRC / "host" / "paged_host.cpp"
+CALL_SRC = CSRC / "host" / "paged_call.cpp"
 HOST_DIR = PKG_DIR / "src" / "cache"
 
 
@@ -85,6 +87,26 @@ def build_host(verbose: bool = False) -> Path:
     cxx = os.environ.get("CXX") or shutil.which("g++") or "g++"
     _run([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Wextra",
           f"-I{sysconfig.get_paths()['include']}", str(HOST_SRC), "-o", str(out) + ".tmp"], verbose)
+    os.replace(str(out) + ".tmp", out)
+    return out
+
+
+def build_call(verbose: bool = False) -> Path:
+    """Compile the native front of the entry points (CPython extension over torch's ATen) to
+    src/kernels/_paged_call<EXT_SUFFIX>; returns its path."""
+    import sysconfig
+
+    import torch
+
+    out = PKG_DIR / "src" / "kernels" / ("_paged_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+    tdir = Path(torch.__file__).resolve().parent
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "g++"
+    _run([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f"-I{sysconfig.get_paths()['include']}", f"-isystem{tdir / 'include'}",
+          f"-isystem{tdir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{INCLUDE}", str(CALL_SRC),
+          f"-L{tdir / 'lib'}", f"-Wl,-rpath,{tdir / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
+          "-o", str(out) + ".tmp"], verbose)
     os.replace(str(out) + ".tmp", out)
     return out
 
@@ -103,8 +125,10 @@ def build(verbose: bool = False) -> Path:
         _run([hipcc, *HIPCC_FLAGS, *incs, "-c", str(src), "-o", str(obj)], verbose)
         return obj
 
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=8) as ex:
+        call = ex.submit(build_call, verbose)
         objs = list(ex.map(compile_one, sources))
+        call.result()
 
     link = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(LIB_PATH) + ".tmp"]
     tlib = _torch_lib_dir()

@@ -175,6 +175,12 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def entry_addresses() -> dict[str, int]:
+    """Entry point -> address in the loaded library."""
+    lib = load()
+    return {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES}
+
+
 def check(status: int, what: str) -> None:
     if status != PA_OK:
         msg = load().pa_last_error_message()

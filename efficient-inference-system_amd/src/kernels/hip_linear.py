@@ -21,7 +21,7 @@ import torch
 import torch.nn as nn
 
 from src.kernels import _lib
-from src.kernels.hip_paged_attention import _stream_ptr
+from src.kernels.hip_paged_attention import _stream_ptr, native_call
 
 MAX_ROWS = 2048  # rows per call accepted by the library
 SUPPORTED_FEATURES = (128, 256, 512, 1024, 2048)
@@ -64,6 +64,12 @@ def linear_rows_hip(x: torch.Tensor, linear: nn.Linear, *, ln: nn.LayerNorm | No
     """out[m] = act(LN(x[m]) W^T + b) + residual[m] for the rows of x (at most 2048); x, the layer's
     parameters, residual and out share one dtype (float32 or bfloat16). copy_to: the same rows are
     also written there (it may be residual itself)."""
+    native = native_call()
+    if native is not None:
+        lw, lb, eps = (ln.weight, ln.bias, ln.eps) if ln is not None else (None, None, 0.0)
+        done = native.linear_rows(x, linear.weight, linear.bias, lw, lb, eps, gelu, residual, out, copy_to)
+        if done is not None:
+            return done
     _rows(x, "x")
     dt = x.dtype
     M, K = x.shape
@@ -155,6 +161,14 @@ def qkv_append_hip(x: torch.Tensor, ln: nn.LayerNorm, attn, k_pool: torch.Tensor
                    slot_mapping: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """q = LN(x) Wq^T + bq for the rows of x; the K and V rows go straight into their pool slots
     (converted to the pool dtype). x, the projections, LayerNorm and q share one dtype."""
+    native = native_call()
+    if native is not None:
+        lw, lb, eps = (ln.weight, ln.bias, ln.eps) if ln is not None else (None, None, 0.0)
+        wq, wk, wv = attn.q_proj, attn.k_proj, attn.v_proj
+        done = native.qkv_append(x, lw, lb, eps, wq.weight, wq.bias, wk.weight, wk.bias, wv.weight, wv.bias,
+                                 k_pool, v_pool, slot_mapping, out)
+        if done is not None:
+            return done
     _rows(x, "x")
     dt = x.dtype
     M, D = x.shape
