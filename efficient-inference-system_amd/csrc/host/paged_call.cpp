@@ -37,7 +37,7 @@ bool ready = false;
 PyObject* workspaces = nullptr;  // {(device index, kind): uint8 tensor}
 PyObject* raw_stream = nullptr;  // torch._C._cuda_getCurrentRawStream
 PyObject* fail = nullptr;        // _lib.check(status, what)
-PyObject* splits = nullptr;      // default_split_blocks(batch, heads, max_pages, device)
+PyObject* splits = nullptr;      // default_split_blocks(batch, heads, max_pages, device, ordered)
 PyObject *kind_decode, *kind_prefill, *str_device;
 
 using Tensor = at::Tensor;
@@ -169,15 +169,19 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (order != nullptr && !(order->scalar_type() == at::kInt && order->is_contiguous())) return nullptr;
     if (a[7] == Py_None) {
       PyObject* dev = PyObject_GetAttr(a[0], str_device);
-      PyObject* sb = dev ? PyObject_CallFunction(splits, "LLLO", (long long)t.B, (long long)t.H, (long long)t.pages, dev) : nullptr;
+      PyObject* sb = dev ? PyObject_CallFunction(splits, "LLLOO", (long long)t.B, (long long)t.H, (long long)t.pages,
+                                                 dev, order ? Py_True : Py_False)
+                         : nullptr;
       Py_XDECREF(dev);
       if (sb == nullptr) return nullptr;
       t.split = PyLong_AsLongLong(sb);
       Py_DECREF(sb);
       if (PyErr_Occurred()) return nullptr;
     }
-    const size_t need = L.decode_ws(t.B, t.H, t.Hd, t.pages, t.split);
-    void* ws = need ? workspace(*t.q, kind_decode, need) : nullptr;
+    const size_t need = t.bs == 16 ? L.decode_ws(t.B, t.H, t.Hd, t.pages, t.split) : 0;
+    Tensor records;  // the balanced launch: this call's own
+    if (need && t.split < 0) records = at::empty({(int64_t)need}, t.q->options().dtype(at::kByte));
+    void* ws = !need ? nullptr : (t.split < 0 ? records.data_ptr() : workspace(*t.q, kind_decode, need));
     void* stream;
     if ((need && ws == nullptr) || !stream_of(*t.q, stream)) return nullptr;
     const Tensor& o = t.result();

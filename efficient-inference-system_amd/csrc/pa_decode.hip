@@ -9,6 +9,7 @@
 // keeps its own online-softmax state (max m, sum l, acc) for the rows it sees, so the inner loop
 // needs no cross-row exchange. Groups merge with shuffles after the loop; wavefronts merge in LDS.
 // The next block's K and V are loaded into a second register set while the current one is used.
+#include <atomic>
 #include <mutex>
 
 #include "pa_attention.h"
@@ -151,6 +152,63 @@ __device__ __forceinline__ void stream_tiles(int cnt, int ids, int tok_base, int
 template <typename IO, bool COH>
 __device__ __forceinline__ void merge_pair(const AttnArgs& a, int bh, int nact, int lane);
 
+// One wavefront's part of a workgroup's KV blocks [jb, je) of request row `pt`, head h, n valid keys:
+// blocks jb + w + k * NW, in chunks of one page-table entry per lane (ids0: the first chunk's entries,
+// loaded ahead by the caller), folded into an online softmax whose state (m, l, acc) goes to LDS.
+template <typename KV, int HD, int NW, int E>
+__device__ __forceinline__ void walk_blocks(const AttnArgs& a, const int32_t* pt, int h, int jb, int je, int n, int ids0,
+                                            int w, int lane, const float (&qv)[E], float (&sm_acc)[NW][HD],
+                                            float (&sm_m)[NW], float (&sm_l)[NW]) {
+  constexpr int BS = 16;
+  using S = DecodeShape<KV, HD, BS>;
+  constexpr int EPL = S::EPL, LPR = S::LPR, R = S::ROUNDS;
+  static_assert(EPL == E, "lane slice");
+  const int r = lane % LPR, g = lane / LPR;
+  float m = kNegBig, l = 0.f;
+  float acc[EPL];
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
+
+  const KV* kpool = static_cast<const KV*>(a.k_pool);
+  const KV* vpool = static_cast<const KV*>(a.v_pool);
+  const int64_t tile_elems = (int64_t)BS * HD;
+  const int64_t head_off = (int64_t)h * tile_elems;
+  const int64_t blk_stride = (int64_t)a.H * tile_elems;
+
+  // This wave's blocks: j = jb + w + k*NW for k < mine, in chunks of one page-table entry per lane.
+  const int span = je - jb;
+  const int mine = span > w ? (span - w + NW - 1) / NW : 0;
+  for (int c0 = 0; c0 < mine; c0 += kWave) {
+    const int cnt = (mine - c0) < kWave ? (mine - c0) : kWave;
+    int ids = -1;
+    if (lane < cnt) ids = c0 == 0 ? ids0 : pt[jb + w + (c0 + lane) * NW];
+    stream_tiles<KV, HD, BS, PA_DECODE_DEPTH, PA_DECODE_NT != 0, R>(
+        cnt, ids, (jb + w + c0 * NW) * BS + g, NW * BS, kpool, vpool, blk_stride, head_off, a.num_blocks, lane,
+        qv, n, m, l, acc);
+  }
+
+  // Merge the TPL lane groups of this wave (lanes with equal r hold the same head_dim slice).
+#pragma unroll
+  for (int off = LPR; off < kWave; off <<= 1) {
+    const float mo = __shfl_xor(m, off);
+    const float lo = __shfl_xor(l, off);
+    const float M = fmaxf(m, mo);
+    const float sa = fast_exp2(m - M), sb = fast_exp2(mo - M);
+    l = l * sa + lo * sb;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) acc[e] = acc[e] * sa + __shfl_xor(acc[e], off) * sb;
+    m = M;
+  }
+  if (g == 0) {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) sm_acc[w][r * EPL + e] = acc[e];
+  }
+  if (lane == 0) {
+    sm_m[w] = m;
+    sm_l[w] = l;
+  }
+}
+
 template <typename KV, typename IO, int HD, int NW>
 __global__ __launch_bounds__(NW * kWave) void decode_fast_kernel(const AttnArgs a) {
   constexpr int BS = 16;
@@ -235,49 +293,7 @@ __global__ __launch_bounds__(NW * kWave) void decode_fast_kernel(const AttnArgs 
   }
 
 
-  float m = kNegBig, l = 0.f;
-  float acc[EPL];
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
-
-  const KV* kpool = static_cast<const KV*>(a.k_pool);
-  const KV* vpool = static_cast<const KV*>(a.v_pool);
-  const int64_t tile_elems = (int64_t)BS * HD;
-  const int64_t head_off = (int64_t)h * tile_elems;
-  const int64_t blk_stride = (int64_t)a.H * tile_elems;
-
-  // This wave's blocks: j = jb + w + k*NW for k < mine, in chunks of one page-table entry per lane.
-  const int span = je - jb;
-  const int mine = span > w ? (span - w + NW - 1) / NW : 0;
-  for (int c0 = 0; c0 < mine; c0 += kWave) {
-    const int cnt = (mine - c0) < kWave ? (mine - c0) : kWave;
-    int ids = -1;
-    if (lane < cnt) ids = c0 == 0 ? ids0 : pt[jb + w + (c0 + lane) * NW];
-    stream_tiles<KV, HD, BS, PA_DECODE_DEPTH, PA_DECODE_NT != 0, R>(
-        cnt, ids, (jb + w + c0 * NW) * BS + g, NW * BS, kpool, vpool, blk_stride, head_off, a.num_blocks, lane,
-        qv, n, m, l, acc);
-  }
-
-  // Merge the TPL lane groups of this wave (lanes with equal r hold the same head_dim slice).
-#pragma unroll
-  for (int off = LPR; off < kWave; off <<= 1) {
-    const float mo = __shfl_xor(m, off);
-    const float lo = __shfl_xor(l, off);
-    const float M = fmaxf(m, mo);
-    const float sa = fast_exp2(m - M), sb = fast_exp2(mo - M);
-    l = l * sa + lo * sb;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] = acc[e] * sa + __shfl_xor(acc[e], off) * sb;
-    m = M;
-  }
-  if (g == 0) {
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) sm_acc[w][r * EPL + e] = acc[e];
-  }
-  if (lane == 0) {
-    sm_m[w] = m;
-    sm_l[w] = l;
-  }
+  walk_blocks<KV, HD, NW>(a, pt, h, jb, je, n, ids0, w, lane, qv, sm_acc, sm_m, sm_l);
   __syncthreads();
 
   float M = kNegBig;
@@ -429,6 +445,176 @@ __global__ __launch_bounds__(kWave) void decode_merge_kernel(const AttnArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
+// Balanced launch: as many workgroups as the compute units hold at once, in gangs of H (member h
+// takes head h, so a gang's workgroups read adjacent slabs of the same blocks, as the kernel above
+// does with heads innermost). The requests' KV blocks, listed request by request (a request without
+// keys counts as one block), are dealt out evenly: gang g takes positions [W g / NG, W (g + 1) / NG)
+// of the list's W, walking the part of every request in its share. A request cut by a share's end
+// leaves one (m, l, acc) record per gang and head, in slot 0 (the share's first request) or 1 (its
+// last), merged in gang order by decode_balanced_merge_kernel; the others are written directly.
+//   bound: HBM. One workgroup per (request, head) leaves the longest contexts running alone at the
+//   end, and a fixed split size costs every batch records and, where the lengths turn out short, empty
+//   workgroups (a second round of them took 5% of a uniform batch). Here the number of pieces is
+//   that of the gangs and every batch ends at once. MI355X, 16 requests x 32 heads x 128 bf16 over
+//   lengths log-uniform in 512 .. 32768, one workgroup per pair -> balanced: 363 -> 324 us (5.8 ->
+//   6.5 TB/s); 64 x 8 heads x 64 fp32 455 -> 307; 16 equal contexts of 32768 1270 -> 1275 (6.8).
+// ---------------------------------------------------------------------------------------------
+constexpr int kBalancedMaxBatch = 512;
+constexpr int kDecodeMergeHd = 128;  // largest head_dim of the fast kernels
+
+// List positions: the blocks request b counts for.
+__device__ __forceinline__ int balanced_blocks(const AttnArgs& a, int b) {
+  int nb = (valid_keys(a.seq_lens[b], a.cur_lens[b], 0) + 15) / 16;
+  nb = nb < a.max_pages ? nb : a.max_pages;
+  return nb > 1 ? nb : 1;
+}
+// Shares of W positions among NG gangs (NG <= W: every share has a position).
+__device__ __forceinline__ int share_start(int W, int NG, int g) { return (int)((int64_t)W * g / NG); }
+// The gang whose share holds position pos: the last g with share_start(g) <= pos.
+__device__ __forceinline__ int share_of(int W, int NG, int pos) {
+  return (int)((((int64_t)pos + 1) * NG - 1) / W);
+}
+
+template <typename KV, typename IO, int HD, int NW>
+__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(sizeof(KV) == 4 && HD == 128 ? 2 : 4)))
+void decode_balanced_kernel(const AttnArgs a) {
+  constexpr int BS = 16;
+  using S = DecodeShape<KV, HD, BS>;
+  constexpr int EPL = S::EPL, LPR = S::LPR;
+  static_assert(NW * kWave >= kBalancedMaxBatch, "one thread per request");
+  __shared__ float sm_acc[NW][HD];
+  __shared__ float sm_m[NW];
+  __shared__ float sm_l[NW];
+  __shared__ int sS[kBalancedMaxBatch + 1];  // list position of each request's first block
+  __shared__ int sWave[NW];
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int gang = blockIdx.x / a.H;
+  const int h = blockIdx.x - gang * a.H;
+  {  // prefix sums: shuffles inside a wavefront, then the wavefronts' totals
+    int x = (int)threadIdx.x < a.B ? balanced_blocks(a, threadIdx.x) : 0;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int y = __shfl_up(x, off);
+      if (lane >= off) x += y;
+    }
+    if (lane == kWave - 1) sWave[w] = x;
+    __syncthreads();
+    for (int ww = 0; ww < w; ++ww) x += sWave[ww];
+    if ((int)threadIdx.x < a.B) sS[threadIdx.x + 1] = x;
+    if (threadIdx.x == 0) sS[0] = 0;
+    __syncthreads();
+  }
+  const int W = __builtin_amdgcn_readfirstlane(sS[a.B]);
+  const int NG = a.num_splits < W ? a.num_splits : W;
+  if (gang >= NG) return;  // uniform over the workgroup
+  const int lo = share_start(W, NG, gang), hi = share_start(W, NG, gang + 1);
+  int b = 0;
+  for (int ub = a.B - 1; b < ub;) {
+    const int mid = (b + ub + 1) / 2;
+    if (__builtin_amdgcn_readfirstlane(sS[mid]) <= lo) b = mid;
+    else ub = mid - 1;
+  }
+  const int r = lane % LPR;
+  for (; b < a.B; ++b) {
+    const int first = __builtin_amdgcn_readfirstlane(sS[b]), end = __builtin_amdgcn_readfirstlane(sS[b + 1]);
+    if (first >= hi) break;
+    const int n = valid_keys(a.seq_lens[b], a.cur_lens[b], 0);
+    const int nb = n > 0 ? end - first : 0;  // (a.max_pages == 0: one position, no block)
+    const int jb = lo > first ? lo - first : 0;
+    int je = hi < end ? hi - first : end - first;
+    je = je < nb ? je : nb;
+    je = je < a.max_pages ? je : a.max_pages;
+    const int32_t* pt = a.page_table + (int64_t)b * a.pt_stride;
+    int ids0 = -1;
+    if (a.max_pages > 0) {
+      const int idx = jb + w + lane * NW;
+      ids0 = pt[idx < a.max_pages ? idx : a.max_pages - 1];
+    }
+    float qv[EPL];
+    const IO* qp = static_cast<const IO*>(a.q) + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + r * EPL;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) qv[e] = Elem<IO>::load(qp + e) * a.scale_log2;
+    walk_blocks<KV, HD, NW>(a, pt, h, jb, je, n, ids0, w, lane, qv, sm_acc, sm_m, sm_l);
+    __syncthreads();
+    const bool whole = lo <= first && hi >= end;
+    float M = kNegBig;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, sm_m[ww]);
+    for (int d = threadIdx.x; d < HD; d += NW * kWave) {
+      float lsum = 0.f, A = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) {
+        const float f = fast_exp2(sm_m[ww] - M);
+        lsum = fmaf(sm_l[ww], f, lsum);
+        A = fmaf(sm_acc[ww][d], f, A);
+      }
+      if (whole) {
+        IO* op = static_cast<IO*>(a.out) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
+        Elem<IO>::store(op + d, lsum > 0.f ? A / lsum : 0.f);
+      } else {
+        float* rec = a.ws + (((int64_t)gang * a.H + h) * 2 + (lo >= first ? 0 : 1)) * (HD + 2);
+        if (d == 0) {
+          rec[0] = M;
+          rec[1] = lsum;
+        }
+        rec[2 + d] = A;
+      }
+    }
+    __syncthreads();  // the next request's states go to the same LDS
+  }
+}
+
+// Merge of the requests cut by the balanced launch: one wavefront per (request, head).
+template <typename IO>
+__global__ __launch_bounds__(kWave) void decode_balanced_merge_kernel(const AttnArgs a) {
+  const int lane = threadIdx.x;
+  const int b = blockIdx.x / a.H, h = blockIdx.x - b * a.H;
+  int before = 0, total = 0, mine = 0;
+  for (int r = lane; r < a.B; r += kWave) {
+    const int p = balanced_blocks(a, r);
+    total += p;
+    before += r < b ? p : 0;
+    mine += r == b ? p : 0;
+  }
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    total += __shfl_xor(total, off);
+    before += __shfl_xor(before, off);
+    mine += __shfl_xor(mine, off);
+  }
+  const int W = __builtin_amdgcn_readfirstlane(total), first = __builtin_amdgcn_readfirstlane(before);
+  const int NG = a.num_splits < W ? a.num_splits : W;
+  const int g0 = share_of(W, NG, first);
+  const int g1 = share_of(W, NG, first + __builtin_amdgcn_readfirstlane(mine) - 1);
+  if (g0 == g1) return;  // written whole
+  const int HD = a.head_dim;
+  const int64_t R = HD + 2;
+  // Gang g's record: slot 0, or 1 where its share starts in an earlier request (only g0's can).
+  auto rec = [&](int g) {
+    return a.ws + (((int64_t)g * a.H + h) * 2 + (share_start(W, NG, g) >= first ? 0 : 1)) * R;
+  };
+  float M = kNegBig;
+  for (int g = g0 + lane; g <= g1; g += kWave) M = fmaxf(M, rec(g)[0]);
+  M = wave_max(M);
+  float lsum = 0.f, A[kDecodeMergeHd / kWave] = {};
+  for (int g = g0; g <= g1; ++g) {
+    const float* x = rec(g);
+    const float f = fast_exp2(x[0] - M);
+    lsum = fmaf(x[1], f, lsum);
+#pragma unroll
+    for (int t = 0; t < kDecodeMergeHd / kWave; ++t)
+      if (lane + t * kWave < HD) A[t] = fmaf(x[2 + lane + t * kWave], f, A[t]);
+  }
+  IO* op = static_cast<IO*>(a.out) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
+  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+#pragma unroll
+  for (int t = 0; t < kDecodeMergeHd / kWave; ++t)
+    if (lane + t * kWave < HD) Elem<IO>::store(op + lane + t * kWave, A[t] * inv);
+}
+
+// ---------------------------------------------------------------------------------------------
 // Generic kernel: one wavefront per (request, head, query row); lanes own head_dim elements and
 // the KV positions are walked one at a time. Serves any block_size and head_dim <= 512, decode
 // or prefill.
@@ -522,12 +708,13 @@ constexpr int kDecodeWaves = PA_DECODE_WAVES;
 
 template <typename KV, typename IO, int HD>
 static void launch_decode_fast(const AttnArgs& a, hipStream_t stream) {
-  int64_t reqs = a.B;
+  int64_t reqs = a.balanced ? 1 : a.B;  // (balanced: num_splits gangs of H workgroups)
 #if PA_DECODE_XCD
   reqs = (reqs + kXcds - 1) / kXcds * kXcds;
 #endif
   const dim3 grid((unsigned)(reqs * a.H * a.num_splits)), block(kDecodeWaves * kWave);
-  decode_fast_kernel<KV, IO, HD, kDecodeWaves><<<grid, block, 0, stream>>>(a);
+  if (a.balanced) decode_balanced_kernel<KV, IO, HD, kDecodeWaves><<<grid, block, 0, stream>>>(a);
+  else decode_fast_kernel<KV, IO, HD, kDecodeWaves><<<grid, block, 0, stream>>>(a);
 }
 
 template <typename IO>
@@ -540,6 +727,40 @@ static bool dispatch_decode_fast_io(const AttnArgs& a, int kv_dtype, hipStream_t
     if (a.head_dim == 128) { launch_decode_fast<uint16_t, IO, 128>(a, stream); return true; }
   }
   return false;
+}
+
+// Gangs of the balanced launch (0: it does not apply): H workgroups each, together no more than the
+// compute units hold at once.
+template <typename KV, typename IO, int HD>
+static int balanced_slots() {  // workgroups per compute unit, per device
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> cached[kMaxDevices];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  int v = cached[dev].load(std::memory_order_relaxed);
+  if (v == 0) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, decode_balanced_kernel<KV, IO, HD, kDecodeWaves>,
+                                                     kDecodeWaves * kWave, 0) != hipSuccess)
+      n = 0;
+    v = n > 0 ? n : -1;
+    cached[dev].store(v, std::memory_order_relaxed);
+  }
+  return v > 0 ? v : 0;
+}
+static int balanced_gangs(int32_t batch, int32_t num_heads, int32_t head_dim, int32_t max_pages, int io_dtype,
+                          int kv_dtype) {
+  if (batch < 1 || batch > kBalancedMaxBatch || max_pages < 1 || (head_dim != 64 && head_dim != 128)) return 0;
+  if ((int64_t)batch * max_pages >= (1LL << 30)) return 0;  // list positions are int
+  const bool kf = kv_dtype == PA_DTYPE_F32, of = io_dtype == PA_DTYPE_F32;
+  int slots;
+  if (head_dim == 64)
+    slots = kf ? (of ? balanced_slots<float, float, 64>() : balanced_slots<float, uint16_t, 64>())
+               : (of ? balanced_slots<uint16_t, float, 64>() : balanced_slots<uint16_t, uint16_t, 64>());
+  else
+    slots = kf ? (of ? balanced_slots<float, float, 128>() : balanced_slots<float, uint16_t, 128>())
+               : (of ? balanced_slots<uint16_t, float, 128>() : balanced_slots<uint16_t, uint16_t, 128>());
+  return (int)((int64_t)slots * pa_host::device_cu_count() / num_heads);
 }
 
 static int num_splits_for(int32_t max_pages, int32_t split_blocks) {
@@ -563,6 +784,16 @@ constexpr int kSameLaunchMaxSplits = 8;
 
 extern "C" size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int32_t head_dim,
                                            int32_t max_pages, int32_t split_blocks) {
+  if (split_blocks < 0) {  // balanced: two records per workgroup, whichever the dtypes
+    if (batch <= 0 || num_heads <= 0) return 0;
+    int g = 0;
+    for (int io = 0; io < 2; ++io)
+      for (int kv = 0; kv < 2; ++kv) {
+        const int x = balanced_gangs(batch, num_heads, head_dim, max_pages, io, kv);
+        g = x > g ? x : g;
+      }
+    return (size_t)g * num_heads * 2 * (head_dim + 2) * sizeof(float);
+  }
   const int s = num_splits_for(max_pages, split_blocks);
   if (s <= 1 || batch <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
   return kDecodeCounterBytes + (size_t)batch * num_heads * s * (head_dim + 2) * sizeof(float);
@@ -607,8 +838,17 @@ static int decode_entry(const void* q, int64_t q_stride_b, int64_t q_stride_h,
   const bool fast = block_size == 16 && (head_dim == 64 || head_dim == 128);
   if (!fast) return launch_generic_attention(a, io_dtype, kv_dtype, stream);
 
+  const int gangs = split_blocks < 0 && workspace != nullptr && !ws_limit_is_scratch
+                        ? balanced_gangs(batch, num_heads, head_dim, max_pages, io_dtype, kv_dtype) : 0;
   const int nsplit = num_splits_for(max_pages, split_blocks);
-  if (nsplit > 1) {
+  if (gangs > 0) {
+    const size_t need = (size_t)gangs * num_heads * 2 * (head_dim + 2) * sizeof(float);
+    if (workspace_bytes < need)
+      PA_FAIL(PA_ERR_WORKSPACE, "decode workspace too small: need %zu bytes, have %zu", need, workspace_bytes);
+    a.num_splits = gangs;
+    a.ws = static_cast<float*>(workspace);
+    a.balanced = 1;
+  } else if (nsplit > 1) {
     const size_t need = pa_decode_workspace_size(batch, num_heads, head_dim, max_pages, split_blocks);
     if (ws_limit_is_scratch && need > workspace_bytes)
       PA_FAIL(PA_ERR_INVALID_ARGUMENT,
@@ -630,7 +870,14 @@ static int decode_entry(const void* q, int64_t q_stride_b, int64_t q_stride_h,
                                            : dispatch_decode_fast_io<uint16_t>(a, kv_dtype, stream);
   if (!ok) PA_FAIL(PA_ERR_UNSUPPORTED, "no decode kernel for head_dim %d", head_dim);
   PA_CHECK_LAUNCH("decode kernel");
-  if (nsplit > 1 && a.counters == nullptr) {
+  if (gangs > 0) {
+    const dim3 grid((unsigned)((int64_t)batch * num_heads)), block(kWave);
+    if (io_dtype == PA_DTYPE_F32)
+      decode_balanced_merge_kernel<float><<<grid, block, 0, stream>>>(a);
+    else
+      decode_balanced_merge_kernel<uint16_t><<<grid, block, 0, stream>>>(a);
+    PA_CHECK_LAUNCH("balanced decode merge kernel");
+  } else if (nsplit > 1 && a.counters == nullptr) {
     const dim3 grid((unsigned)((int64_t)batch * num_heads)), block(kWave);
     if (io_dtype == PA_DTYPE_F32)
       decode_merge_kernel<float><<<grid, block, 0, stream>>>(a);

@@ -76,7 +76,12 @@ def _workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
     return ws
 
 
-def default_split_blocks(batch: int, num_heads: int, max_pages: int, device: torch.device) -> int:
+# split_blocks value asking pa_decode for its balanced launch (see include/paged_hip.h).
+DECODE_BALANCED = -1
+
+
+def default_split_blocks(batch: int, num_heads: int, max_pages: int, device: torch.device,
+                         ordered: bool = False) -> int:
     """KV blocks per decode split: 0 (no split) when (request, head) pairs alone fill the GPU or
     the context is at most 256 tokens; 16 blocks when contexts are at most 1024 tokens and the
     pairs fill at most one workgroup per compute unit (at most 4 splits, merged inside the launch:
@@ -84,9 +89,20 @@ def default_split_blocks(batch: int, num_heads: int, max_pages: int, device: tor
     7.8-8.1 us split); otherwise enough splits for about two workgroups per compute unit, 16 to
     32 blocks each when there are at most 128 pairs, at least 16 blocks above that. Measured
     (graph replay, MI355X): 1-4 requests x 32 heads x 128 bf16 at 8k tokens 26 / 36 / 64 us with
-    32-block splits against 74 / 75 / 83 us unsplit."""
+    32-block splits against 74 / 75 / 83 us unsplit.
+
+    DECODE_BALANCED above 128 pairs where contexts may pass 8192 tokens: it ends every workgroup at
+    once whatever the lengths. Against the rules above, heads x head_dim, lengths log-uniform / equal:
+    16 x 32 x 128 bf16 to 32k 363 -> 324 us / 1270 -> 1275; 64 x 32 x 128, bf16 KV, to 32k 1360 -> 1226;
+    8 x 32 x 128 to 32k 188 -> 155, to 8k 57 -> 53 / 168 -> 170; 64 x 8 x 64 fp32 to 32k 455 -> 307;
+    32 x 8 x 64 fp32 to 32k 313 -> 160; 20 x 8 x 64, bf16 KV, to 32k 83 -> 57 / at 8k 57 -> 58. At 4096
+    tokens its second launch (4.5 us) takes what it gains (equal lengths 163 -> 168, others within
+    1%), and with eight pairs per compute unit in the caller's order (longest first) the grid's end
+    is already filled with short contexts (1214 against 1226)."""
     units = batch * num_heads
     target = 2 * cu_count(device)
+    if units > 128 and max_pages >= 512 and batch <= 512 and not (ordered and units >= 4 * target):
+        return DECODE_BALANCED
     if units == 0 or units >= target or max_pages <= 16:
         return 0
     if max_pages <= 64:
@@ -196,10 +212,14 @@ def paged_attention_decode_hip(
     max_pages = page_table.shape[1] if page_table.dim() == 2 else 0
     pt_stride = page_table.stride(0) if page_table.dim() == 2 and B > 0 else max_pages
     if split_blocks is None:
-        split_blocks = default_split_blocks(B, H, max_pages, q.device)
+        split_blocks = default_split_blocks(B, H, max_pages, q.device, order is not None)
     lib = _lib.load()
-    ws_bytes = lib.pa_decode_workspace_size(B, H, Hd, max_pages, split_blocks)
-    ws_ptr = _workspace(q.device, ws_bytes, "decode").data_ptr() if ws_bytes else None
+    ws_bytes = lib.pa_decode_workspace_size(B, H, Hd, max_pages, split_blocks) if bs == 16 else 0
+    ws = None
+    if ws_bytes:  # (the balanced launch: records only, this call's own)
+        ws = _workspace(q.device, ws_bytes, "decode") if split_blocks > 0 else \
+            torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+    ws_ptr = ws.data_ptr() if ws is not None else None
     status = lib.pa_decode(
         q.data_ptr(), q.stride(0), q.stride(1),
         out.data_ptr(), out.stride(0), out.stride(1), _lib.dtype_code(q.dtype),

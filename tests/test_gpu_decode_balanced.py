@@ -1,0 +1,106 @@
+"""The balanced decode launch (split_blocks = DECODE_BALANCED): workgroup gangs share all requests' KV
+blocks evenly, cutting requests anywhere. Against the unsplit launch and the oracle."""
+import math
+
+import pytest
+import torch
+
+import oracle
+from src.kernels import _lib
+from src.kernels.hip_paged_attention import DECODE_BALANCED, default_split_blocks, paged_attention_decode_hip
+
+pytestmark = pytest.mark.gpu
+
+
+def _batch(device, lens, H, Hd, io, kv, seed=0, extra_pages=3):
+    g = torch.Generator().manual_seed(seed)
+    counts = [-(-n // 16) for n in lens]
+    N = sum(counts) + 5
+    perm = torch.randperm(N, generator=g).to(torch.int32)
+    table = torch.full((len(lens), max(counts) + extra_pages), -1, dtype=torch.int32)
+    lists, at = [], 0
+    for b, c in enumerate(counts):
+        lists.append(perm[at:at + c].tolist())
+        table[b, :c] = perm[at:at + c]
+        at += c
+    q = torch.randn(len(lens), 1, H, Hd, generator=g).to(io).transpose(1, 2)
+    k, v = (torch.randn(N, H, 16, Hd, generator=g).to(kv) for _ in range(2))
+    seq = torch.tensor(lens, dtype=torch.int32)
+    return (q, k, v, table, seq, torch.ones_like(seq)), lists
+
+
+LENS = [[1], [4000], [0, 0, 0], [0, 5, 0, 300, 16, 17], [16] * 70, [2000, 1, 1, 1, 900], list(range(1, 513)),
+        [333] * 31 + [7000]]
+
+
+@pytest.mark.parametrize("io,kv", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
+                                   (torch.bfloat16, torch.bfloat16)], ids=["fp32", "bf16kv", "bf16"])
+@pytest.mark.parametrize("H,Hd", [(8, 64), (32, 128), (3, 64)])
+@pytest.mark.parametrize("lens", LENS, ids=lambda x: f"{len(x)}x{max(x)}")
+def test_same_as_unsplit(device, lens, H, Hd, io, kv):
+    print(f"balanced decode {lens[:6]} H {H} Hd {Hd} {io} {kv}", flush=True)
+    args, lists = _batch(device, lens, H, Hd, io, kv)
+    dev = [t.to(device) for t in args]
+    want = paged_attention_decode_hip(*dev, split_blocks=0).float()
+    out = torch.full_like(dev[0], 9.0)
+    got = paged_attention_decode_hip(*dev, split_blocks=DECODE_BALANCED, out=out).float()
+    # fp32 sums in another order (values of N(0, 1) averaged: at most a few ulp of 1); bf16 outputs may
+    # round to the neighbour, 2^-8 of their size
+    bound = 4e-6 if io == torch.float32 else 2.0**-8 * float(want.abs().max()) + 4e-6
+    assert float((got - want).abs().max()) <= bound
+    if len(lens) < 40 and max(lens) <= 4000:
+        ref = oracle.paged_attention(*(x.float() for x in args[:3]), lists, lens, [1] * len(lens))
+        assert float((got.cpu() - torch.as_tensor(ref)).abs().max()) <= (1e-4 if io == torch.float32 else 2e-2)
+
+
+def test_two_streams_and_graph_replays(device):
+    """Each call takes its own records: calls on two streams at once, and a captured call replayed between
+    eager ones, give what they give alone."""
+    cases = [_batch(device, lens, 32, 128, torch.float32, torch.bfloat16, seed)[0]
+             for seed, lens in ((1, [9000, 30, 700, 2500]), (2, [64, 12000, 5000]))]
+    cases = [[t.to(device) for t in c] for c in cases]
+    call = lambda c, **kw: paged_attention_decode_hip(*c, split_blocks=DECODE_BALANCED, **kw)  # noqa: E731
+    want = [call(c).clone() for c in cases]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(10):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got[i].append(call(cases[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(g, want[i]) for g in got[i])
+    out = torch.empty_like(want[0])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(cases[0], out=out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        other = call(cases[1])
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[0]) and torch.equal(other, want[1])
+
+
+def test_limits(device):
+    """More requests than one workgroup lists, another block size, or no workspace: the call runs unsplit."""
+    lib = _lib.load()
+    assert lib.pa_decode_workspace_size(513, 8, 64, 600, DECODE_BALANCED) == 0
+    assert lib.pa_decode_workspace_size(8, 8, 96, 600, DECODE_BALANCED) == 0
+    assert lib.pa_decode_workspace_size(8, 1 << 20, 64, 600, DECODE_BALANCED) == 0
+    assert default_split_blocks(513, 8, 600, device) == 0 and default_split_blocks(64, 8, 600, device) == DECODE_BALANCED
+    assert default_split_blocks(64, 32, 600, device, True) == 0
+    args, _ = _batch(device, [5] * 600, 2, 64, torch.float32, torch.float32)
+    dev = [t.to(device) for t in args]
+    assert torch.equal(paged_attention_decode_hip(*dev, split_blocks=DECODE_BALANCED),
+                       paged_attention_decode_hip(*dev, split_blocks=0))
+    q, k, v, table, seq, cur = dev = [t.to(device) for t in _batch(device, [300, 9], 8, 64, torch.float32, torch.float32)[0]]
+    want, out = paged_attention_decode_hip(*dev, split_blocks=0), torch.empty_like(q)
+    for fn, tail in ((lib.pa_decode, (None, 0)), (lib.pa_decode_noalloc, ())):
+        out.fill_(9.0)
+        st = fn(q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(), out.stride(0), out.stride(1), 0, k.data_ptr(),
+                v.data_ptr(), 0, k.shape[0], table.data_ptr(), table.stride(0), table.shape[1], seq.data_ptr(),
+                cur.data_ptr(), None, 2, 8, 64, 16, 1 / math.sqrt(64), DECODE_BALANCED, *tail,
+                torch.cuda.current_stream().cuda_stream)
+        assert st == 0 and torch.equal(out, want)
