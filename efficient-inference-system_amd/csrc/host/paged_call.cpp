@@ -207,6 +207,7 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* ws = need ? workspace(*t.q, kind_prefill, need) : nullptr;
     void* stream;
     if ((need && ws == nullptr) || !stream_of(*t.q, stream)) return nullptr;
+    if (need && stream != nullptr) return nullptr;  // (the kept workspace is the default stream's)
     const Tensor& o = t.result();
     const int st = unlocked([&] {
       return L.prefill(t.q->data_ptr(), t.q->stride(0), t.q->stride(1), t.q->stride(2), o.data_ptr(), o.stride(0),

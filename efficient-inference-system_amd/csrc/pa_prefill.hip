@@ -643,42 +643,69 @@ static bool prefill_fast_shape(int32_t head_dim, int32_t block_size) {
   return block_size == 16 && (head_dim == 64 || head_dim == 128);
 }
 
-// Kernel choice between the wide-tile kernel (128 query rows per workgroup) and the 16-row one, by
-// the wide kernel's unit count U = B * H * ceil(T / 128) against the CU count. The wide kernel
-// shares each staged KV step among 128 rows but needs enough units to fill the GPU: it is taken
-// from U >= 2 CUs always, for bf16 KV from U >= 3/4 of the CUs, and for fp32 KV at head_dim 128
-// from U >= CUs (the crossovers measured on MI355X). PAGED_HIP_PREFILL_KERNEL=wide / tile forces
-// one of them (tests use it to cover both at small sizes).
-static bool use_wide_prefill(int kv_dtype, int32_t head_dim, int32_t batch, int32_t num_heads, int32_t query_len) {
-  const char* env = getenv("PAGED_HIP_PREFILL_KERNEL");
-  if (env != nullptr && strcmp(env, "wide") == 0) return true;
-  if (env != nullptr && strcmp(env, "tile") == 0) return false;
-  const int64_t units = prefill_wide_units(batch, num_heads, query_len);
-  const int64_t cus = pa_host::device_cu_count();
-  if (units >= 2 * cus) return true;
-  if (kv_dtype == PA_DTYPE_BF16) return 4 * units >= 3 * cus;
-  return head_dim == 128 && units >= cus;
+}  // namespace pa (the choice is declared in pa_attention.h)
+
+// Kernel of an unsplit (or balanced) prefill call: the one with the least estimated time
+//   fixed + p * max(alone, rate * units * 256 / CUs, reads * KV bytes of a page / 6 TB/s)
+// in us, p the page table's width. `alone` is one page of a workgroup that has its compute unit for
+// itself, `rate` a page of one unit when all compute units are shared, units the kernel's own:
+// (request, head) pairs times 128-row tiles (wide, balanced), 16-row tiles (16-row kernel) or 32-row
+// tiles (split-step). Fitted on MI355X to 675 shapes: 1-64 requests of 32 heads x 128 or 8 heads x
+// 64, chunks of 16-512 rows, contexts to 60-6000 tokens spread over a factor 4, fp32 and bf16 KV; the
+// choice is within 1% of the best of them in the mean and takes 7-16% off the rules by unit counts
+// that it replaces. What those missed: short chunks in 128-row tiles (fp32, 8 x 32 heads x 128, 16
+// rows over 1.5k: wide 156 us, 16-row 45; 64 x 8 x 64, 16 rows 105 / 45), one to two 128-row tiles
+// per compute unit over long contexts (fp32, 8 x 32 x 128, 128 rows over 6k: wide 600, balanced 392;
+// 8 x 8 x 64, 512 rows 358 / 190, bf16 94 / 55) and few rows over long contexts at head_dim 64
+// (bf16, 4 x 8 heads, 64 rows over 6k: 16-row 29, split-step 20; fp32, 1 x 8: 16-row 53, balanced 37).
+// The lines that the estimates do not draw:
+//   - balanced up to two tiles per compute unit (beyond, the tiles fill the grid's end by themselves:
+//     fp32, 32 x 8 x 64, 512 rows over 1.5k 231 wide, 274 balanced) and, at head_dim 64 with at most
+//     half a tile per compute unit, from 192 pages (below, gains and losses are a few us);
+//   - split-step below three quarters of a 128-row tile per compute unit (no measurement beyond).
+pa::PrefillKind pa::prefill_choice(int kv_dtype, int32_t head_dim, int32_t batch, int32_t num_heads,
+                                   int32_t query_len, int32_t max_pages, bool balanced) {
+  struct Fit {
+    double fixed, alone, rate, reads;
+  };
+  const bool f32 = kv_dtype == PA_DTYPE_F32;
+  const bool wide_rows = head_dim == 128;
+  const Fit kWide = f32 ? (wide_rows ? Fit{4, 1.72, .0037, 1.1} : Fit{5, .91, .0021, 1.1})
+                        : (wide_rows ? Fit{4, .36, .0007, 1.1} : Fit{3, .25, .0005, 1.1});
+  const Fit kBal = f32 ? (wide_rows ? Fit{26, .34, .0040, 1.15} : Fit{20, .13, .00185, 1.15})
+                       : (wide_rows ? Fit{28, .075, .0009, 1.15} : Fit{14, .04, .00042, 1.15});
+  Fit kTile = f32 ? (wide_rows ? Fit{7, .35, .00125, 1.0} : Fit{4, .19, .00052, 1.0})
+                  : (wide_rows ? Fit{5, .10, .00032, 1.0} : Fit{3, .115, .00016, 1.0});
+  const Fit kSplit = {5.2, .05, .00025, 1.2};
+  const int64_t cus = pa_host::device_cu_count() > 0 ? pa_host::device_cu_count() : 256;
+  const int64_t pairs = (int64_t)batch * num_heads;
+  const int64_t u128 = pairs * ((query_len + 127) / 128), u32 = pairs * ((query_len + 31) / 32),
+                u16 = pairs * ((query_len + 15) / 16);
+  if (u16 > u128) kTile.reads = 1.3;  // (several tiles read a page, from L2 at best)
+  const double page_us = 0.65 * pairs * head_dim * 16 * 2 * (f32 ? 4 : 2) / 6e6;
+  auto cost = [&](const Fit& f, int64_t units) {
+    double page = f.alone;
+    const double shared = f.rate * units * 256.0 / cus, read = f.reads * page_us;
+    page = page > shared ? page : shared;
+    page = page > read ? page : read;
+    return f.fixed + page * max_pages;
+  };
+  PrefillKind best = PrefillKind::kWide;
+  double least = cost(kWide, u128);
+  auto offer = [&](PrefillKind k, double c) {
+    if (c < least) {
+      least = c;
+      best = k;
+    }
+  };
+  offer(PrefillKind::kTile, cost(kTile, u16));
+  if (balanced && u128 <= 2 * cus && (head_dim == 128 || 2 * u128 > cus || max_pages >= 192))
+    offer(PrefillKind::kBalanced, cost(kBal, u128));
+  if (!f32 && head_dim == 64 && 4 * u128 < 3 * cus) offer(PrefillKind::kSplit, cost(kSplit, u32));
+  return best;
 }
 
-// Split-step kernel (32-row tiles, 8 wavefronts splitting the KV steps; bf16 KV at head_dim 64)
-// instead of the 16-row kernel, by its unit count U = B * H * ceil(T / 32) (one workgroup per CU
-// at most) and the page-table width: it is taken for chunks longer than 64 rows from half the CUs
-// to the CU count, and up to twice the CU count (two rounds) once the widest request spans 96
-// pages, where it measured faster on MI355X (its 32-row tiles read each KV step half as often as
-// the 16-row kernel's, which pays once the context outweighs the second round's tail: at 512
-// units 0.96-1.02x of the 16-row time at 48-64 pages, 0.74-0.87x from 96 pages; at 384 units a
-// tie at 88-96 pages, 0.92-0.97x from 120); below half the CUs or for short chunks the 16-row
-// kernel's extra workgroups win. PAGED_HIP_PREFILL_KERNEL=split forces it where it applies (tile
-// forces the 16-row kernel).
-static bool use_split_prefill(int32_t batch, int32_t num_heads, int32_t query_len, int32_t max_pages) {
-  const char* env = getenv("PAGED_HIP_PREFILL_KERNEL");
-  if (env != nullptr && strcmp(env, "split") == 0) return true;
-  if (env != nullptr && strcmp(env, "tile") == 0) return false;
-  const int64_t units = prefill_split_units(batch, num_heads, query_len);
-  const int64_t cus = pa_host::device_cu_count();
-  if (query_len <= 64 || 2 * units < cus) return false;
-  return units <= cus || (units <= 2 * cus && max_pages >= 96);
-}
+namespace pa {
 
 static int prefill_num_splits(int32_t max_pages, int32_t split_blocks) {
   if (split_blocks <= 0 || max_pages <= split_blocks) return 1;
@@ -750,12 +777,18 @@ extern "C" int pa_prefill(const void* q, int64_t q_stride_b, int64_t q_stride_h,
       return launch_prefill_wide(a, io_dtype, kv_dtype, stream);
     }
   }
-  if (split_blocks <= 0 && prefill_wide_supported(kv_dtype, head_dim, block_size) &&
-      use_wide_prefill(kv_dtype, head_dim, batch, num_heads, query_len))
-    return launch_prefill_wide(a, io_dtype, kv_dtype, stream);
-  if (split_blocks <= 0 && prefill_split_supported(kv_dtype, head_dim, block_size) &&
-      use_split_prefill(batch, num_heads, query_len, max_pages))
-    return launch_prefill_split(a, io_dtype, stream);
+  if (split_blocks <= 0) {
+    // PAGED_HIP_PREFILL_KERNEL = wide / split / tile forces one where it applies (tests cover each).
+    PrefillKind kind = prefill_choice(kv_dtype, head_dim, batch, num_heads, query_len, max_pages, false);
+    if (const char* env = getenv("PAGED_HIP_PREFILL_KERNEL")) {
+      if (strcmp(env, "wide") == 0) kind = PrefillKind::kWide;
+      if (strcmp(env, "split") == 0 && prefill_split_supported(kv_dtype, head_dim, block_size)) kind = PrefillKind::kSplit;
+      if (strcmp(env, "tile") == 0) kind = PrefillKind::kTile;
+    }
+    if (kind == PrefillKind::kWide && prefill_wide_supported(kv_dtype, head_dim, block_size))
+      return launch_prefill_wide(a, io_dtype, kv_dtype, stream);
+    if (kind == PrefillKind::kSplit) return launch_prefill_split(a, io_dtype, stream);
+  }
 
   const int64_t units = (int64_t)batch * num_heads * ((query_len + 15) / 16);
   const int nsplit = prefill_num_splits(max_pages, split_blocks);

@@ -733,7 +733,7 @@ void prefill_wide_kernel(const AttnArgs a) {
 //   in the bf16 kernel. The next step's fp32 values wait in registers meanwhile, so one LDS stage
 //   (48 KB at head_dim 128) is enough and two workgroups share a compute unit.
 //   error: the scores' leading products are accumulated apart from the rest, in 8 (not 64) rounded
-//   additions, an output in 12 (not 16) per 32 keys. 4 x 32 heads x 128, 512-token chunks over
+//   additions, an output in 12 (not 16) per 32 keys, at head_dim 64 in one. 4 x 32 heads x 128, 512-token chunks over
 //   1-4k, N(0, 1): 8e-7 of the output's norm against float64; fp32 MFMA 1e-6.
 //   measured (MI355X, the same shape, chunk append included): 948 -> 605 us; at 4k contexts 185
 //   TFLOP/s, 55% MFMA and 31% VALU busy at a clock that the load pulls down to 1.75 GHz (all-zero
@@ -1062,10 +1062,12 @@ void prefill_wide_f32_kernel(const AttnArgs a) {
     sacc += rest;
   };
   // O^T += V^T P^T: slice mm contracts keys 16mm + 8jj + 4*G2 + r at slot (G2, 4jj + r), the lane's
-  // registers 8mm + 4jj + r; small partial products first. At raised wavefront priority, as in the
-  // bf16 kernel.
+  // registers 8mm + 4jj + r; small partial products first. At head_dim 64, where registers allow, a
+  // step's products are summed from zero and added to the output once: one addition rounded at the
+  // output's size per 32 keys, not 12. At raised wavefront priority, as in the bf16 kernel.
   auto weigh = [&]() {
     __builtin_amdgcn_s_setprio(1);
+    bf16x8 pp[2][3];
 #pragma unroll
     for (int mm = 0; mm < 2; ++mm) {
       u32x4 w1, w2, w3;
@@ -1075,25 +1077,40 @@ void prefill_wide_f32_kernel(const AttnArgs a) {
         split_bf16x3(sacc[8 * mm + 2 * e], sacc[8 * mm + 2 * e + 1], p1, p2, p3);
         w1[e] = p1; w2[e] = p2; w3[e] = p3;
       }
-      const bf16x8 p1 = __builtin_bit_cast(bf16x8, w1), p2 = __builtin_bit_cast(bf16x8, w2),
-                   p3 = __builtin_bit_cast(bf16x8, w3);
+      pp[mm][0] = __builtin_bit_cast(bf16x8, w1);
+      pp[mm][1] = __builtin_bit_cast(bf16x8, w2);
+      pp[mm][2] = __builtin_bit_cast(bf16x8, w3);
+    }
+    auto add = [&](f32x16& o, int mm, int d) {
+      const uint16_t* vp = sbuf + 3 * PLANE + v_off(d) + 16 * mm * HD;
+      auto part = [&](const uint16_t* x) {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(x));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(x + 8 * HD));
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      };
+      const bf16x8 v1 = part(vp), v2 = part(vp + PLANE), v3 = part(vp + 2 * PLANE);
+      o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v3, pp[mm][0], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, pp[mm][2], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, pp[mm][1], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, pp[mm][0], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, pp[mm][1], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, pp[mm][0], o, 0, 0, 0);
+    };
+    if constexpr (HD == 64) {
 #pragma unroll
       for (int d = 0; d < DU; ++d) {
-        const uint16_t* vp = sbuf + 3 * PLANE + v_off(d) + 16 * mm * HD;
-        auto part = [&](const uint16_t* x) {
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(x));
-          const s16x4 hi =
-              __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(x + 8 * HD));
-          return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        };
-        const bf16x8 v1 = part(vp), v2 = part(vp + PLANE), v3 = part(vp + 2 * PLANE);
-        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v3, p1, oacc[d], 0, 0, 0);
-        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p3, oacc[d], 0, 0, 0);
-        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, p2, oacc[d], 0, 0, 0);
-        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, p1, oacc[d], 0, 0, 0);
-        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p2, oacc[d], 0, 0, 0);
-        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p1, oacc[d], 0, 0, 0);
+        f32x16 t;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) t[e] = 0.f;
+        add(t, 0, d);
+        add(t, 1, d);
+        oacc[d] += t;
       }
+    } else {
+#pragma unroll
+      for (int mm = 0; mm < 2; ++mm)
+#pragma unroll
+        for (int d = 0; d < DU; ++d) add(oacc[d], mm, d);
     }
     __builtin_amdgcn_s_setprio(0);
   };
@@ -1651,50 +1668,11 @@ int64_t prefill_balanced_grid(int32_t batch, int32_t num_heads, int32_t query_le
   // products per query row as a 32-key step at 128).
   const int nbs = head_dim == 64 && kv_dtype == PA_DTYPE_BF16 ? 2 * kWideNsub64 : 2;
   const int64_t cus = pa_host::device_cu_count();
-  // Where it pays (MI355X, head_dim 128, graph-free eager timings; default launch -> balanced):
-  // few tiles over long contexts, where the default launch leaves CUs idle or each tile walks
-  // hundreds of steps alone. bf16 KV: 1 x 32 heads, 512-token chunk over 8k 159 -> 96 us, over 3k
-  // 81 -> 59 us; 2 x 32, 256-token chunks over 8k 208 -> 103 us; 1 x 32, 128-token chunk over 16k
-  // 130 -> 86 us; it loses on short contexts (1 x 32, 128-token chunk over 4k 31 -> 38 us; 256
-  // over 2k 28 -> 34 us) and on grids of two or more tiles per CU (8 x 32 heads, 512-token chunks:
-  // 237 -> 250 us), and ties in between (256 tiles: 0 to -5%). fp32 KV (a step costs more, so
-  // cutting pays sooner): 1 x 32, 512-token chunk over 8k 807 -> 574 us, over 1k 144 -> 126 us;
-  // 256-token chunk over 2k 109 -> 105 us; 128-token chunk over 16k 356 -> 321 us, over 4k 92 ->
-  // 108 us (loses). So: at most half a tile per CU and at least 8192 tile-steps (tiles x the
-  // longest tile's 32-key steps, from the page table's width), 4096 for fp32 KV from a quarter
-  // tile per CU; two workgroups per CU unless that cuts a tile more than 8 ways (then one).
-  const int64_t steps = ((int64_t)max_pages + nbs - 1) / nbs;
-  const int64_t min_steps = kv_dtype == PA_DTYPE_F32 && 4 * units >= cus ? 4096 : 8192;
-  bool pays = 2 * units <= cus && units * steps >= min_steps;
-  // Head_dim 64 (bf16 KV, 64-key steps: twice the softmax work per matrix product of a head_dim 128
-  // step, and the split-step kernel as the alternative): 1 x 32 heads, 512-token chunk over 8k
-  // 64.6 -> 56.9 us, 2 x 32, 256 over 8k 63.8 -> 57.3 us, 1 x 32, 128 over 16k 52.8 -> 46.8 us;
-  // ties at 1 x 32, 512 over 4k (38.8 / 38.1) and 1 x 8, 512 over 8k (32.2 / 31.4); loses at
-  // 1 x 16, 512 over 8k (33.1 -> 38.1), 4 x 8, 256 over 4k (19.3 -> 28.5) and 1 x 32, 512 over 2k
-  // (25.1 -> 28.8). So at least 16384 tile-steps, or 256 steps (16k keys) per tile.
-  if (head_dim == 64 && kv_dtype == PA_DTYPE_BF16) pays = 2 * units <= cus && (units * steps >= 16384 || steps >= 256);
-  int per_cu = 4 * units >= cus ? 2 : 1;  // two per CU cut each tile into 2 cus / units pieces
-  // Head_dim 64, fp32 KV (32-key steps; the alternative is the 16-row kernel, whose B * H *
-  // ceil(T / 16) workgroups leave CUs idle when tiles are few): 1 x 8 heads, 128-token chunk over
-  // 32k 369.6 -> 126.2 us, over 8k 94.5 -> 54.7 us (one workgroup per CU); 512 over 16k 209.2 ->
-  // 173.3 us, 1 x 32, 128 over 16k 190.8 -> 169.8 us, 1 x 32, 512 over 8k 351.7 -> 307.1 us,
-  // 2 x 32, 256 over 8k 354.1 -> 306.6 us (two per CU); ties at 1 x 16, 256 over 8k (98.0 / 98.2)
-  // and 1 x 8, 512 over 8k (113.0 / 104.9); loses at 4 x 8, 256 over 4k (79.9 -> 97.1), 2 x 8,
-  // 512 over 4k (83.7 -> 96.6), 1 x 32, 512 over 2k (99.6 -> 102.6) and 4 x 8, 256 over 768
-  // (23.4 -> 33.9). Checked on further shapes: 1 x 8, 256 over 16k 187.6 -> 107.9 us, 2 x 8, 128
-  // over 16k 186.2 -> 109.6 us, 1 x 8, 512 over 32k 371.0 -> 302.5 us, 2 x 16, 512 over 8k 340.0 ->
-  // 307.5 us, 1 x 32, 512 over 4k 180.4 -> 171.6 us; but 1 x 32, 256 over 8k 151.1 -> 165.9 us and
-  // 1 x 64, 128 over 8k 153.2 -> 176.7 us lose: there the 16-row kernel has two workgroups per
-  // CU, its LDS-staged build at its best. So at least 16384 tile-steps unless the 16-row grid
-  // holds one to two workgroups per CU, or 256 steps per tile at most one tile per 16 CUs; two
-  // workgroups per CU from one tile per 8 CUs.
-  if (head_dim == 64 && kv_dtype == PA_DTYPE_F32) {
-    const int64_t rows16 = (int64_t)batch * num_heads * ((query_len + 15) / 16);
-    const bool rows16_at_best = rows16 > cus && rows16 <= 2 * cus;
-    pays = 2 * units <= cus &&
-           ((units * steps >= 16384 && !rows16_at_best) || (steps >= 256 && 16 * units <= cus));
-    per_cu = 8 * units >= cus ? 2 : 1;
-  }
+  bool pays = prefill_choice(kv_dtype, head_dim, batch, num_heads, query_len, max_pages, true) == PrefillKind::kBalanced;
+  // Two workgroups per CU unless that cuts a tile more than 8 ways (then one); for fp32 KV at head_dim
+  // 64 from one tile per 8 CUs (1 x 8 heads, 512-token chunk over 16k, 209.2 -> 173.3 us with two).
+  int per_cu = 4 * units >= cus ? 2 : 1;
+  if (head_dim == 64 && kv_dtype == PA_DTYPE_F32) per_cu = 8 * units >= cus ? 2 : 1;
   if (!pays && units > 2 * cus) per_cu = slots;
   if (const char* env = getenv("PAGED_HIP_PREFILL_BALANCE")) {
     if (strcmp(env, "force") == 0) pays = true;

@@ -80,6 +80,20 @@ def _workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
 DECODE_BALANCED = -1
 
 
+PREFILL_COUNTER_BYTES = 64 << 10  # PA_PREFILL_COUNTER_BYTES in include/paged_hip.h
+
+
+def _prefill_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
+    """A prefill call's workspace: the kept one on the default stream, where calls follow each other;
+    on other streams, and so under capture, the call's own (its arrival counters zeroed), so that calls
+    on several streams and replays of several graphs never share counters or records."""
+    if _stream_ptr(device) == 0:
+        return _workspace(device, nbytes, "prefill")
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    ws[:PREFILL_COUNTER_BYTES].zero_()
+    return ws
+
+
 def default_split_blocks(batch: int, num_heads: int, max_pages: int, device: torch.device,
                          ordered: bool = False) -> int:
     """KV blocks per decode split: 0 (no split) when (request, head) pairs alone fill the GPU or
@@ -274,7 +288,8 @@ def paged_attention_prefill_hip(
         split_blocks = default_prefill_split_blocks(B, H, T, max_pages, q.device, k_pool.dtype)
     lib = _lib.load()
     ws_bytes = lib.pa_prefill_workspace_size(B, H, T, Hd, max_pages, split_blocks) if bs == 16 else 0
-    ws_ptr = _workspace(q.device, ws_bytes, "prefill").data_ptr() if ws_bytes else None
+    ws = _prefill_workspace(q.device, ws_bytes) if ws_bytes else None
+    ws_ptr = ws.data_ptr() if ws is not None else None
     status = lib.pa_prefill(
         q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
         out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), _lib.dtype_code(q.dtype),

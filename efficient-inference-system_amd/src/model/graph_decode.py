@@ -329,10 +329,10 @@ class _Captured:
             self.split_blocks = default_prefill_split_blocks(B, H, Tb, pages, device, pools[0].dtype)
             ws_bytes = lib.pa_prefill_workspace_size(B, H, Tb, Hd, pages, self.split_blocks)
         # Allocated outside the capture and referenced here, so the address the graph records
-        # stays valid for the graph's lifetime.
-        # (A balanced decode takes its records from the graph's own pool.)
-        kept = ws_bytes and (Tb > 1 or self.split_blocks > 0)
-        self.ws = _workspace(device, ws_bytes, "decode" if Tb == 1 else "prefill") if kept else None
+        # stays valid for the graph's lifetime. (Prefill calls and a balanced decode take theirs from
+        # the graph's own pool.)
+        kept = ws_bytes and Tb == 1 and self.split_blocks > 0
+        self.ws = _workspace(device, ws_bytes, "decode") if kept else None
         self.fused = B * Tb <= FUSED_STEP_ROWS and fused_decode_enabled() and hip_linear.model_supported(model)
         # Steps of at most 16 rows of an fp32 model (every decode step at batch <= 16): per layer
         # four launches, the MLP in one (fc1 column tiles adding their fc2 shares with atomic adds).
