@@ -37,6 +37,22 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// fp32 products on the bf16 matrix cores: an fp32 operand as the sum of three bf16 parts, a product
+// as the six partial products of parts whose indices add up to at most 4. Values from kSplitMax on
+// (infinities among them) have no such split whose products stay finite.
+constexpr float kSplitMax = 1152921504606846976.f;  // 2^60
+
+// Two fp32 values as packed bf16 triples: x = w1 + w2 + w3, each part the nearest bf16 of the rest.
+__device__ __forceinline__ void split_bf16x3(float lo, float hi, uint32_t& w1, uint32_t& w2, uint32_t& w3) {
+  w1 = pack_bf16x2(lo, hi);
+  lo -= bf16_lo(w1);
+  hi -= bf16_hi(w1);
+  w2 = pack_bf16x2(lo, hi);
+  lo -= bf16_lo(w2);
+  hi -= bf16_hi(w2);
+  w3 = pack_bf16x2(lo, hi);
+}
+
 template <typename T> struct Elem;
 template <> struct Elem<float> {
   __device__ static __forceinline__ float load(const float* p) { return *p; }

@@ -779,6 +779,320 @@ __global__ __launch_bounds__(kTileWaves * kWave) void tile_linear_kernel(const L
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Block kernel for LayerNorm layers over many rows: a workgroup owns a 128-row x 64-column output tile,
+// one 32 x 32 block per wavefront, and walks K in chunks of BK through two LDS stages of bf16
+// operands on v_mfma_f32_32x32x16_bf16. The tiled kernel normalises its 32 rows for every 32
+// columns; here the statistics and the normalised operand serve 64 columns of 128 rows.
+//   fp32: every operand is the sum of three bf16 parts and every product its six leading partial
+//   products (split_bf16x3), the leading one accumulated apart from the others (error 1.7e-7 of the
+//   norm at K 512, fp32 MFMA 2.4e-7). The fp32 MFMA runs at 1/16 of the bf16 rate and bounded the
+//   tiled kernel; six bf16 products take 6/16 of its time. Values of 2^60 and more (infinities among
+//   them) have no split with finite products: a workgroup that meets one forms its tile again with
+//   v_mfma_f32_32x32x2_f32 on operands from memory.
+//   bf16: one plane, the operands as they are.
+//   bound: LDS, which serves each wavefront 6 KB per six MFMAs (its peak), and the latency of a
+//   chunk: 1.6k cycles of which the MFMAs take 768.
+// The values of the next chunks wait in a ring of register sets, four chunks ahead (a chunk is
+// multiplied in less than the memory's latency); the conversion (LayerNorm, split) and LDS stores of
+// the next one are issued between the MFMAs, and one barrier per chunk publishes them. Each row's
+// statistics come from one read of the row held in registers (mean first, then the biased variance
+// of the deviations).
+// ---------------------------------------------------------------------------------------------
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kBlockK = 512;  // features
+constexpr int kBlockRows = 128, kBlockCols = 64;
+
+template <typename T>
+struct BlockShape {
+  static constexpr int BM = kBlockRows, BN = kBlockCols, BK = sizeof(T) == 2 ? 64 : 32;
+  static constexpr bool BF = sizeof(T) == 2;
+  static constexpr int NW = (BM / 32) * (BN / 32);       // wavefronts
+  static constexpr int NT = NW * kWave;
+  static constexpr int NP = BF ? 1 : 3;                  // planes
+  static constexpr int PLANE = (BM + BN) * BK;           // elements per plane: A rows, then B rows
+  static constexpr int EP = 16 / (int)sizeof(T);         // values per 16-byte piece
+  static constexpr int PPR = BK / EP;                    // pieces per row and chunk
+  static constexpr int PA = BM * PPR / NT, PB = BN * PPR / NT;  // pieces per thread
+  static_assert(PA * NT == BM * PPR && PB * NT == BN * PPR && NT % PPR == 0, "pieces");
+  static_assert(BK % 16 == 0 && BK <= 128 && kBlockK % BK == 0, "slices");
+};
+
+template <typename T>
+__global__ __launch_bounds__(BlockShape<T>::NT) __attribute__((amdgpu_waves_per_eu(2)))
+void block_linear_kernel(const LinArgs a) {
+  using Sh = BlockShape<T>;
+  constexpr int BM = Sh::BM, BN = Sh::BN, BK = Sh::BK;
+  constexpr bool BF = Sh::BF;
+  constexpr int NT = Sh::NT, NP = Sh::NP, PLANE = Sh::PLANE, EP = Sh::EP, PPR = Sh::PPR, PA = Sh::PA, PB = Sh::PB;
+  constexpr int CPR = BK / 8;     // 16-byte chunks per row of a plane
+  constexpr int RPB = 128 / BK;   // rows of a plane per 256 bytes (one pass over the banks)
+  constexpr int WN = BN / 32;
+  constexpr int D = 4;            // register sets
+  __shared__ __attribute__((aligned(16))) uint16_t stage0[2 * NP * PLANE];
+  __shared__ float sm_stat[BM][2];
+  __shared__ u32x4 sm_ln[2][kBlockK / EP];
+  __shared__ int sm_bad;
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int G2 = lane >> 5, c = lane & 31;
+  const int wn = w % WN, wm = w / WN;
+  const int tiles_per_seg = (a.seg_n + BN - 1) / BN;
+  const int seg = blockIdx.x / tiles_per_seg;
+  const int n0 = (blockIdx.x - seg * tiles_per_seg) * BN;
+  const int r0 = blockIdx.y * BM;
+  const T* W = static_cast<const T*>(seg == 0 ? a.w[0] : (seg == 1 ? a.w[1] : a.w[2]));
+  const T* X = static_cast<const T*>(a.x);
+  constexpr int nch = kBlockK / BK;
+  if (threadIdx.x == 0) sm_bad = 0;
+  static_assert(kBlockK / EP <= NT, "one LayerNorm piece per thread");
+  if (threadIdx.x < kBlockK / EP) {
+    sm_ln[0][threadIdx.x] = static_cast<const u32x4*>(a.ln_w)[threadIdx.x];
+    sm_ln[1][threadIdx.x] = static_cast<const u32x4*>(a.ln_b)[threadIdx.x];
+  }
+
+  // This thread's pieces: A rows (tid + n NT) / PPR, columns EP * (tid % PPR) of every chunk; B alike.
+  // Rows past M and columns past the layer repeat the last one and are never stored.
+  const int pr = threadIdx.x / PPR, pc = threadIdx.x % PPR;
+  const T *pa[PA], *pb[PB];
+#pragma unroll
+  for (int n = 0; n < PA; ++n) {
+    const int r = r0 + pr + n * (NT / PPR);
+    pa[n] = X + (int64_t)(r < a.M ? r : a.M - 1) * a.x_stride + EP * pc;
+  }
+#pragma unroll
+  for (int n = 0; n < PB; ++n) {
+    const int r = n0 + pr + n * (NT / PPR);
+    pb[n] = W + (int64_t)(r < a.seg_n ? r : a.seg_n - 1) * a.K + EP * pc;
+  }
+  struct Pieces {
+    u32x4 a[PA], b[PB];
+  };
+  Pieces ring[D];  // chunk ch in set ch % D
+  auto load = [&](Pieces& r, int ch) {
+#pragma unroll
+    for (int n = 0; n < PA; ++n) r.a[n] = *reinterpret_cast<const u32x4*>(pa[n] + ch * BK);
+#pragma unroll
+    for (int n = 0; n < PB; ++n) r.b[n] = *reinterpret_cast<const u32x4*>(pb[n] + ch * BK);
+  };
+  load(ring[0], 0);
+
+  // ---- LayerNorm statistics: TPR threads per row, 16-byte pieces -------------------------------
+  {
+    constexpr int TPR = NT / BM;      // threads per row
+    constexpr int PCS = kBlockK / (EP * TPR);
+    static_assert(TPR == 4, "threads per row");
+    const int row = threadIdx.x / TPR, tp = threadIdx.x % TPR;
+    const u32x4* xp = reinterpret_cast<const u32x4*>(X + (int64_t)(r0 + row < a.M ? r0 + row : a.M - 1) * a.x_stride);
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
+    auto add = [&](const u32x4& q, float center, bool square) {
+      const uint32_t qw[4] = {q[0], q[1], q[2], q[3]};
+#pragma unroll
+      for (int e = 0; e < EP; ++e) {
+        const float d = LinT<T>::get(qw, e) - center;
+        part[e & 3] = square ? fmaf(d, d, part[e & 3]) : part[e & 3] + d;
+      }
+    };
+    auto total = [&]() {
+      const float t = group_sum<TPR>((part[0] + part[1]) + (part[2] + part[3])) / kBlockK;
+      part[0] = part[1] = part[2] = part[3] = 0.f;
+      return t;
+    };
+    u32x4 xr[PCS];
+#pragma unroll
+    for (int t = 0; t < PCS; ++t) xr[t] = xp[t * TPR + tp];
+#pragma unroll
+    for (int t = 0; t < PCS; ++t) add(xr[t], 0.f, false);
+    const float mean = total();
+#pragma unroll
+    for (int t = 0; t < PCS; ++t) add(xr[t], mean, true);
+    const float var = total();
+    if (tp == 0) {
+      sm_stat[row][0] = mean;
+      sm_stat[row][1] = 1.f / sqrtf(var + a.ln_eps);
+    }
+    __syncthreads();
+  }
+  float mu[PA], rs[PA];
+#pragma unroll
+  for (int n = 0; n < PA; ++n) {
+    mu[n] = sm_stat[pr + n * (NT / PPR)][0];
+    rs[n] = sm_stat[pr + n * (NT / PPR)][1];
+  }
+  auto swz = [](int r) { return (r / RPB) & (CPR - 1); };
+  float mx = 0.f;
+  // Convert the pieces of chunk ch and store them into stage st.
+  auto store = [&](const Pieces& rs_, int ch, uint16_t* st) {
+    const u32x4 rg = sm_ln[0][ch * PPR + pc], rbe = sm_ln[1][ch * PPR + pc];
+    auto put = [&](const u32x4& q, int r, bool norm, float m_, float r_) {
+      const uint32_t qw[4] = {q[0], q[1], q[2], q[3]};
+      uint16_t* row = st + r * BK;
+      if constexpr (BF) {
+        u32x4 o = q;
+        if (norm) {
+          const uint32_t gw[4] = {rg[0], rg[1], rg[2], rg[3]}, bw[4] = {rbe[0], rbe[1], rbe[2], rbe[3]};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            o[e] = pack_bf16x2(fmaf((LinT<T>::get(qw, 2 * e) - m_) * r_, LinT<T>::get(gw, 2 * e), LinT<T>::get(bw, 2 * e)),
+                               fmaf((LinT<T>::get(qw, 2 * e + 1) - m_) * r_, LinT<T>::get(gw, 2 * e + 1),
+                                    LinT<T>::get(bw, 2 * e + 1)));
+        }
+        *reinterpret_cast<u32x4*>(row + 8 * (pc ^ swz(r))) = o;
+      } else {
+        float f[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f[e] = __uint_as_float(qw[e]);
+          if (norm) f[e] = fmaf((f[e] - m_) * r_, __uint_as_float(rg[e]), __uint_as_float(rbe[e]));
+        }
+        mx = fmaxf(fmaxf(mx, fabsf(f[0])), fabsf(f[1]));
+        mx = fmaxf(fmaxf(mx, fabsf(f[2])), fabsf(f[3]));
+        uint32_t lo[3], hi[3];
+        split_bf16x3(f[0], f[1], lo[0], lo[1], lo[2]);
+        split_bf16x3(f[2], f[3], hi[0], hi[1], hi[2]);
+        uint16_t* d = row + 8 * ((pc >> 1) ^ swz(r)) + 4 * (pc & 1);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) *reinterpret_cast<u32x2*>(d + p * PLANE) = u32x2{lo[p], hi[p]};
+      }
+    };
+#pragma unroll
+    for (int n = 0; n < PA; ++n) put(rs_.a[n], pr + n * (NT / PPR), true, mu[n], rs[n]);
+#pragma unroll
+    for (int n = 0; n < PB; ++n) put(rs_.b[n], BM + pr + n * (NT / PPR), false, 0.f, 0.f);
+  };
+
+  f32x16 acc, rest;  // products of the leading parts; the other partial products (fp32)
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = rest[e] = 0.f;
+  auto multiply = [&](const uint16_t* st) {
+    const int ar = 32 * wm + c, br = BM + 32 * wn + c;
+#pragma unroll
+    for (int s0 = 0; s0 < BK / 16; ++s0) {
+      const int q = 2 * s0 + G2;
+      const uint16_t* ap = st + ar * BK + 8 * (q ^ swz(ar));
+      const uint16_t* bp = st + br * BK + 8 * (q ^ swz(br));
+      bf16x8 av[NP], bv[NP];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        av[p] = *reinterpret_cast<const bf16x8*>(ap + p * PLANE);
+        bv[p] = *reinterpret_cast<const bf16x8*>(bp + p * PLANE);
+      }
+      if constexpr (!BF) {
+        rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[2], bv[0], rest, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[0], acc, 0, 0, 0);
+        rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[2], rest, 0, 0, 0);
+        rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1], bv[1], rest, 0, 0, 0);
+        rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1], bv[0], rest, 0, 0, 0);
+        rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[1], rest, 0, 0, 0);
+      } else {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[0], acc, 0, 0, 0);
+      }
+    }
+  };
+
+  // ---- K walk: chunk ch is multiplied from stage ch & 1 while chunk ch + 1 goes into the other -----
+  store(ring[0], 0, stage0);
+  // Iteration ch: chunks ch + 1 .. ch + D - 1 are on their way into the register sets. Loads and
+  // stores are unconditional (past the last chunk they repeat it, into a stage that is not read), so
+  // that the compiler's wait counts are exact and the later chunks' loads stay in flight.
+  auto clamp = [&](int ch) { return ch < nch ? ch : nch - 1; };
+#pragma unroll
+  for (int d = 1; d < D; ++d) load(ring[d], clamp(d));
+  auto iteration = [&](auto dc, int ch) {
+    constexpr int d = decltype(dc)::value;
+    static_assert(D % 2 == 0, "stage ch & 1 is stage d & 1");
+    uint16_t* cur = stage0 + (d & 1) * NP * PLANE;
+    uint16_t* nxt = stage0 + ((d & 1) ^ 1) * NP * PLANE;
+    __syncthreads();  // chunk ch is published; every wavefront is past chunk ch - 1
+    load(ring[d], clamp(ch + D));
+    multiply(cur);
+    store(ring[(d + 1) % D], clamp(ch + 1), nxt);
+    if constexpr (!BF) {
+      // one MFMA, then a share of the conversion that fits its 32 cycles
+#pragma unroll
+      for (int g = 0; g < 6 * (BK / 16); ++g) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+      }
+    }
+  };
+  static_assert(nch % D == 0, "whole rounds of the ring");
+  for (int ch0 = 0; ch0 < nch; ch0 += D) static_for<0, D>([&](auto dc) { iteration(dc, ch0 + decltype(dc)::value); });
+  if constexpr (!BF) {
+    if (mx >= kSplitMax) sm_bad = 1;
+    acc += rest;
+  }
+  __syncthreads();  // stages are free; sm_bad is published
+  if constexpr (!BF) {
+    if (__builtin_amdgcn_readfirstlane(sm_bad) != 0) {
+      // fp32 products, operands from memory: MFMA slot G2 of index k is feature k + G2
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+      const int m = r0 + 32 * wm + c, n = n0 + 32 * wn + c;
+      const float* xp = reinterpret_cast<const float*>(X) + (int64_t)(m < a.M ? m : a.M - 1) * a.x_stride + G2;
+      const float* wp = reinterpret_cast<const float*>(W) + (int64_t)(n < a.seg_n ? n : a.seg_n - 1) * a.K + G2;
+#pragma unroll 1
+      for (int k = 0; k < kBlockK; k += 2) {
+        const float x = fmaf((xp[k] - sm_stat[32 * wm + c][0]) * sm_stat[32 * wm + c][1],
+                             static_cast<const float*>(a.ln_w)[k + G2], static_cast<const float*>(a.ln_b)[k + G2]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, wp[k], acc, 0, 0, 0);
+      }
+    }
+  }
+  // ---- epilogue: lane (G2, c) holds rows 8j + 4 G2 + r of column c of its block ------------------
+  const int n = n0 + 32 * wn + c;
+  if (n >= a.seg_n) return;
+  const float bias = a.b[seg] != nullptr ? Elem<T>::load(static_cast<const T*>(a.b[seg]) + n) : 0.f;
+  auto row = [&](int e) { return r0 + 32 * wm + 8 * (e >> 2) + 4 * G2 + (e & 3); };
+  auto in = [&](int e) { return row(e) < a.M ? row(e) : a.M - 1; };
+  if (a.act == 1) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float v = acc[e] + bias;
+      acc[e] = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] += bias;
+  }
+  // (every load of a group goes out before the first is used: rows past M read row M - 1)
+  if (a.k_pool != nullptr && seg > 0) {
+    int slot[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) slot[e] = a.slots[in(e)];
+    const int h = n / a.Hd, dd = n - h * a.Hd;
+    void* pool = seg == 1 ? a.k_pool : a.v_pool;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const uint32_t blk = (uint32_t)slot[e] / (uint32_t)a.bs;
+      if (row(e) >= a.M || slot[e] < 0 || (int64_t)blk >= a.num_blocks) continue;
+      const int64_t off = (((int64_t)blk * a.H + h) * a.bs + (slot[e] - (int)blk * a.bs)) * a.Hd + dd;
+      if (a.pool_bf16) static_cast<uint16_t*>(pool)[off] = f32_to_bf16(acc[e]);
+      else static_cast<float*>(pool)[off] = acc[e];
+    }
+    return;
+  }
+  if (a.res != nullptr) {
+    const T* rp = static_cast<const T*>(a.res) + seg * a.seg_n + n;
+    float res[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) res[e] = Elem<T>::load(rp + in(e) * a.res_stride);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] += res[e];
+  }
+  T* op = static_cast<T*>(a.out) + seg * a.seg_n + n;
+  T* cp = static_cast<T*>(a.out_copy) + seg * a.seg_n + n;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    if (row(e) >= a.M) continue;
+    Elem<T>::store(op + row(e) * a.out_stride, acc[e]);
+    if (a.out_copy != nullptr) Elem<T>::store(cp + row(e) * a.out_copy_stride, acc[e]);
+  }
+}
+
 #ifndef PA_LIN_FORCE_CW_LOG2
 #define PA_LIN_FORCE_CW_LOG2 0
 #endif
@@ -864,7 +1178,32 @@ static int launch_tile_linear(const LinArgs& a, hipStream_t stream) {
   return PA_OK;
 }
 
+static int launch_block_linear(const LinArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)(a.nseg * ((a.seg_n + kBlockCols - 1) / kBlockCols)),
+                  (unsigned)((a.M + kBlockRows - 1) / kBlockRows));
+  if (a.bf16) block_linear_kernel<uint16_t><<<grid, BlockShape<uint16_t>::NT, 0, stream>>>(a);
+  else block_linear_kernel<float><<<grid, BlockShape<float>::NT, 0, stream>>>(a);
+  PA_CHECK_LAUNCH("block linear kernel");
+  return PA_OK;
+}
+
+// The block kernel instead of the tiled one: LayerNorm layers of 512 features whose tiled grid
+// (32 x 32 outputs) has more than four and a half workgroups per compute unit. Its workgroups take
+// 14 (bf16) or 22 us whether one or one per compute unit runs; the tiled kernel's time grows with its
+// grid. Graph replay on MI355X, tiled / block, us: fc1 (2048 columns) fp32 20.5 / 22.3 at 512 rows,
+// 30.5 / 23.1 at 768, 38.8 / 24.3 at 1024, bf16 13.8 / 14.1, 19.7 / 14.3, 24.8 / 14.8; q/k/v (1536) fp32
+// 17.9 / 21 at 512, 25.7 / 22.3 at 768, 31.1 / 22.4 at 1024, bf16 14.1 / 13.2, 18.9 / 13.5, 21.6 / 13.6.
+// Layers without LayerNorm stay: K 512 fp32 8.8 / 15.7 at 1024 rows, K 2048 23.2 / 47.5.
+static bool use_block_linear(const LinArgs& a) {
+  if (a.row_sel != nullptr || a.token_keys != nullptr || a.ln_w == nullptr || a.K != kBlockK) return false;
+  const char* env = getenv("PAGED_HIP_LINEAR_KERNEL");
+  if (env != nullptr) return strcmp(env, "block") == 0;
+  const int64_t tiled = (int64_t)a.nseg * ((a.seg_n + 31) / 32) * ((a.M + 31) / 32);
+  return 2 * tiled >= 9 * (int64_t)pa_host::device_cu_count();
+}
+
 static int launch_small_linear(LinArgs a, hipStream_t stream) {
+  if (use_block_linear(a)) return launch_block_linear(a, stream);
   if (use_tile_linear(a)) return launch_tile_linear(a, stream);
   a.cw_log2 = lin_cw_log2(a);
   const int64_t tiles = (int64_t)a.nseg * ((a.seg_n + (1 << a.cw_log2) - 1) >> a.cw_log2);

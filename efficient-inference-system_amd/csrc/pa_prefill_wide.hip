@@ -743,19 +743,6 @@ void prefill_wide_kernel(const AttnArgs a) {
 // wavefront whose q or whose workgroup's K or V held one walks its steps a second time, with
 // v_mfma_f32_32x32x2_f32 on operands read straight from memory (slow; fp32 products as they are).
 // NaN needs no care: its parts are NaN.
-constexpr float kSplitMax = 1152921504606846976.f;  // 2^60
-
-// Two fp32 values as packed bf16 triples: x = w1 + w2 + w3, each part the nearest bf16 of the rest.
-__device__ __forceinline__ void split_bf16x3(float lo, float hi, uint32_t& w1, uint32_t& w2, uint32_t& w3) {
-  w1 = pack_bf16x2(lo, hi);
-  lo -= bf16_lo(w1);
-  hi -= bf16_hi(w1);
-  w2 = pack_bf16x2(lo, hi);
-  lo -= bf16_lo(w2);
-  hi -= bf16_hi(w2);
-  w3 = pack_bf16x2(lo, hi);
-}
-
 template <typename IO, int HD, bool BAL>
 __global__ __launch_bounds__(kWideWaves * kWave) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_wide_f32_kernel(const AttnArgs a) {

@@ -78,18 +78,18 @@ T_BUCKETS = (16, 32, 64, 96, 128, 160, 192, 224, 256)
 # Largest step (rows = B * bucketed T) for which each fused launch beats torch's layers, per
 # dtype. Measured in HIP-graph replay on MI355X (fused vs torch, us), d_model 512, d_ff 2048,
 # vocab 5000, with the library's choice between its 16-row and tiled kernels:
-#   LayerNorm + q/k/v + append  fp32 11.8 at 256 rows, 32.5 vs 40.4 at 1024, 47.2 vs 46.4 at 1536
-#                               (torch without the append); bf16 22.1 vs 33.4 at 1024
+#   LayerNorm + q/k/v + append  fp32 11.8 at 256 rows, 22.9 vs 40.4 at 1024 (torch without the
+#                               append); bf16 13.5 vs 33.4 at 1024
 #   out_proj + residual         fp32 8.6 vs 11.0 at 1024, 12.6 vs 13.0 at 1536; bf16 5.0 vs 8.0 at 1024
-#   LayerNorm + fc1 + GELU      fp32 29.4 vs 31.4 at 768, 39.0 vs 33.6 at 1024; bf16 13.5 vs 14.5
-#                               at 512, 19.4 vs 16.7 at 768
+#   LayerNorm + fc1 + GELU      fp32 23.6 vs 32.2 at 768, 24.7 vs 32.0 at 1024; bf16 13.1 vs 14.8
+#                               at 512, 14.1 vs 17.7 at 1024
 #   fc2 + residual              fp32 23.7 vs 24.0 at 1024, 34.3 vs 31.9 at 1536; bf16 10.6 vs 11.0
 #                               at 1024, 15.5 vs 12.7 at 1536
 #   LayerNorm + lm_head         fp32 10.7 vs 11.8 at 48, 15.8 vs 11.8 at 64; bf16 9.1 vs 10.4 at 64,
 #                               13.6 vs 11.2 at 96
 FUSED_ROWS = {
-    torch.float32: {"qkv": 1024, "out_proj": 1024, "fc1": 768, "fc2": 1024, "lm_head": 48},
-    torch.bfloat16: {"qkv": 1024, "out_proj": 1024, "fc1": 512, "fc2": 1024, "lm_head": 64},
+    torch.float32: {"qkv": 1024, "out_proj": 1024, "fc1": 1024, "fc2": 1024, "lm_head": 48},
+    torch.bfloat16: {"qkv": 1024, "out_proj": 1024, "fc1": 1024, "fc2": 1024, "lm_head": 64},
 }
 FUSED_STEP_ROWS = 1024  # steps above this run the torch layers throughout
 
