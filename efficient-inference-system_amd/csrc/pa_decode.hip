@@ -775,12 +775,17 @@ using namespace pa;
 // Split workspace layout: arrival counters (one int32 per (request, head), at most
 // kDecodeCounterBytes / 4 pairs) at the start, zero between calls, then the split records. The
 // counters region has one fixed size whatever the call's shape, so calls of any shapes can share
-// a workspace and always find their counters at zero.
+// a workspace and always find their counters at zero. The balanced launch's records lie behind that
+// region too, which it neither reads nor writes.
 constexpr size_t kDecodeCounterBytes = PA_DECODE_COUNTER_BYTES;
 // Splits per (request, head) up to which the last split to finish merges the records in the same
 // launch; more splits are merged by a second launch (its merge reads them faster than one
 // workgroup's device-scope loads).
 constexpr int kSameLaunchMaxSplits = 8;
+
+static size_t balanced_workspace(int gangs, int32_t num_heads, int32_t head_dim) {
+  return gangs > 0 ? kDecodeCounterBytes + (size_t)gangs * num_heads * 2 * (head_dim + 2) * sizeof(float) : 0;
+}
 
 extern "C" size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int32_t head_dim,
                                            int32_t max_pages, int32_t split_blocks) {
@@ -792,7 +797,7 @@ extern "C" size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int
         const int x = balanced_gangs(batch, num_heads, head_dim, max_pages, io, kv);
         g = x > g ? x : g;
       }
-    return (size_t)g * num_heads * 2 * (head_dim + 2) * sizeof(float);
+    return balanced_workspace(g, num_heads, head_dim);
   }
   const int s = num_splits_for(max_pages, split_blocks);
   if (s <= 1 || batch <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
@@ -842,11 +847,11 @@ static int decode_entry(const void* q, int64_t q_stride_b, int64_t q_stride_h,
                         ? balanced_gangs(batch, num_heads, head_dim, max_pages, io_dtype, kv_dtype) : 0;
   const int nsplit = num_splits_for(max_pages, split_blocks);
   if (gangs > 0) {
-    const size_t need = (size_t)gangs * num_heads * 2 * (head_dim + 2) * sizeof(float);
+    const size_t need = balanced_workspace(gangs, num_heads, head_dim);
     if (workspace_bytes < need)
       PA_FAIL(PA_ERR_WORKSPACE, "decode workspace too small: need %zu bytes, have %zu", need, workspace_bytes);
     a.num_splits = gangs;
-    a.ws = static_cast<float*>(workspace);
+    a.ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + kDecodeCounterBytes);
     a.balanced = 1;
   } else if (nsplit > 1) {
     const size_t need = pa_decode_workspace_size(batch, num_heads, head_dim, max_pages, split_blocks);

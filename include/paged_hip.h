@@ -76,8 +76,9 @@ const char* pa_last_error_message(void);
  * split_blocks < 0 asks for the balanced launch (at most 512 requests; other calls run unsplit): as many
  * workgroups as the GPU holds share the requests' KV blocks evenly whatever their lengths, and a
  * second kernel merges the requests that a share's end cuts. Its workspace of
- * pa_decode_workspace_size() bytes holds records only: it needs no initial state and may be freed or
- * reused, in stream order, after the call. Without a workspace such a call runs unsplit. order is
+ * pa_decode_workspace_size() bytes holds records behind PA_DECODE_COUNTER_BYTES that it leaves
+ * alone: it needs no initial state, may be freed or reused, in stream order, after the call, and, if
+ * zeroed once, serves split calls (split_blocks > 0) as well, in any order. Without a workspace such a call runs unsplit. order is
  * not used.
  *
  * order: optional int32 [B] permutation giving the processing order of requests (e.g. longest
@@ -92,10 +93,10 @@ int pa_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h,
               float scale, int32_t split_blocks,
               void* workspace, size_t workspace_bytes, void* stream);
 
-/* Bytes of workspace pa_decode needs for these sizes (split_blocks < 0: two records per workgroup of
- * the balanced launch on the current device, 0 where it does not apply; otherwise 0 when split_blocks
- * == 0 or no request can need more than one split, else PA_DECODE_COUNTER_BYTES + 4 * batch * num_heads * splits *
- * (head_dim + 2)). No reference counterpart: the Triton decode path has no split-K.
+/* Bytes of workspace pa_decode needs for these sizes (split_blocks < 0: PA_DECODE_COUNTER_BYTES and two
+ * records per workgroup of the balanced launch on the current device, 0 where it does not apply;
+ * otherwise 0 when split_blocks == 0 or no request can need more than one split, else
+ * PA_DECODE_COUNTER_BYTES + 4 * batch * num_heads * splits * (head_dim + 2)). No reference counterpart: the Triton decode path has no split-K.
  * Calls that share a workspace must not run concurrently (e.g. on different streams). */
 size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int32_t head_dim,
                                 int32_t max_pages, int32_t split_blocks);

@@ -104,3 +104,33 @@ def test_limits(device):
                 cur.data_ptr(), None, 2, 8, 64, 16, 1 / math.sqrt(64), DECODE_BALANCED, *tail,
                 torch.cuda.current_stream().cuda_stream)
         assert st == 0 and torch.equal(out, want)
+
+
+def _entry(lib, dev, out, split, ws, nbytes):
+    """pa_decode itself, on a workspace of the caller's."""
+    q, k, v, table, seq, cur = dev
+    B, H, _, Hd = q.shape
+    return lib.pa_decode(q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(), out.stride(0), out.stride(1),
+                         _lib.dtype_code(q.dtype), k.data_ptr(), v.data_ptr(), _lib.dtype_code(k.dtype), k.shape[0],
+                         table.data_ptr(), table.stride(0), table.shape[1], seq.data_ptr(), cur.data_ptr(), None,
+                         B, H, Hd, 16, 1 / math.sqrt(Hd), split, ws.data_ptr(), nbytes,
+                         torch.cuda.current_stream().cuda_stream)
+
+
+@pytest.mark.parametrize("io,kv", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)],
+                         ids=["fp32", "bf16"])
+def test_one_workspace_for_balanced_and_split_calls(device, io, kv):
+    """A workspace zeroed once serves balanced and split calls in any order: the balanced launch's records
+    stay clear of the arrival counters, which are zero after every call."""
+    lib = _lib.load()
+    dev = [t.to(device) for t in _batch(device, [900, 40, 1000], 8, 64, io, kv)[0]]
+    sizes = [lib.pa_decode_workspace_size(3, 8, 64, dev[3].shape[1], s) for s in (DECODE_BALANCED, 16)]
+    assert min(sizes) > 0
+    ws = torch.zeros(max(sizes), dtype=torch.uint8, device=device)
+    want = paged_attention_decode_hip(*dev, split_blocks=0).float()
+    bound = 4e-6 if io == torch.float32 else 2.0**-8 * float(want.abs().max()) + 4e-6  # (as above)
+    for split in (DECODE_BALANCED, 16, 16, DECODE_BALANCED, 16):
+        out = torch.full_like(dev[0], 9.0)
+        assert _entry(lib, dev, out, split, ws, ws.numel()) == 0
+        assert float((out.float() - want).abs().max()) <= bound, split
+        assert int(torch.count_nonzero(ws[:256 << 10])) == 0, split
