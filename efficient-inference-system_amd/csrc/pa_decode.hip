@@ -843,13 +843,13 @@ static int decode_entry(const void* q, int64_t q_stride_b, int64_t q_stride_h,
   const bool fast = block_size == 16 && (head_dim == 64 || head_dim == 128);
   if (!fast) return launch_generic_attention(a, io_dtype, kv_dtype, stream);
 
-  const int gangs = split_blocks < 0 && workspace != nullptr && !ws_limit_is_scratch
-                        ? balanced_gangs(batch, num_heads, head_dim, max_pages, io_dtype, kv_dtype) : 0;
+  int gangs = 0;
+  if (split_blocks < 0 && workspace != nullptr && !ws_limit_is_scratch) {
+    gangs = balanced_gangs(batch, num_heads, head_dim, max_pages, io_dtype, kv_dtype);
+    if (workspace_bytes < balanced_workspace(gangs, num_heads, head_dim)) gangs = 0;  // unsplit
+  }
   const int nsplit = num_splits_for(max_pages, split_blocks);
   if (gangs > 0) {
-    const size_t need = balanced_workspace(gangs, num_heads, head_dim);
-    if (workspace_bytes < need)
-      PA_FAIL(PA_ERR_WORKSPACE, "decode workspace too small: need %zu bytes, have %zu", need, workspace_bytes);
     a.num_splits = gangs;
     a.ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + kDecodeCounterBytes);
     a.balanced = 1;

@@ -78,8 +78,8 @@ const char* pa_last_error_message(void);
  * second kernel merges the requests that a share's end cuts. Its workspace of
  * pa_decode_workspace_size() bytes holds records behind PA_DECODE_COUNTER_BYTES that it leaves
  * alone: it needs no initial state, may be freed or reused, in stream order, after the call, and, if
- * zeroed once, serves split calls (split_blocks > 0) as well, in any order. Without a workspace such a call runs unsplit. order is
- * not used.
+ * zeroed once, serves split calls (split_blocks > 0) as well, in any order. Without a workspace, or
+ * with a smaller one, such a call runs unsplit. The balanced launch does not use order.
  *
  * order: optional int32 [B] permutation giving the processing order of requests (e.g. longest
  * first, for load balance); NULL means 0..B-1. Results do not depend on it.

@@ -134,3 +134,17 @@ def test_one_workspace_for_balanced_and_split_calls(device, io, kv):
         assert _entry(lib, dev, out, split, ws, ws.numel()) == 0
         assert float((out.float() - want).abs().max()) <= bound, split
         assert int(torch.count_nonzero(ws[:256 << 10])) == 0, split
+
+
+def test_a_workspace_too_small_for_the_records_runs_unsplit(device):
+    """As without a workspace: the balanced launch is a wish, whatever memory comes with the call."""
+    lib = _lib.load()
+    dev = [t.to(device) for t in _batch(device, [900, 40, 1000], 8, 64, torch.float32, torch.float32)[0]]
+    need = lib.pa_decode_workspace_size(3, 8, 64, dev[3].shape[1], DECODE_BALANCED)
+    assert need > 0
+    ws = torch.zeros(need, dtype=torch.uint8, device=device)
+    want = paged_attention_decode_hip(*dev, split_blocks=0)
+    for nbytes in (0, 4096, 256 << 10):
+        out = torch.full_like(dev[0], 9.0)
+        assert _entry(lib, dev, out, DECODE_BALANCED, ws, nbytes) == 0, lib.pa_last_error_message()
+        assert torch.equal(out, want) and int(torch.count_nonzero(ws)) == 0
