@@ -37,6 +37,7 @@ bool ready = false;
 PyObject* workspaces = nullptr;  // {(device index, kind): uint8 tensor}
 PyObject* raw_stream = nullptr;  // torch._C._cuda_getCurrentRawStream
 PyObject* fail = nullptr;        // _lib.check(status, what)
+PyObject* side_workspace = nullptr;  // _call_workspace(device, bytes, kind): off the default stream
 PyObject* splits = nullptr;      // default_split_blocks(batch, heads, max_pages, device, ordered)
 PyObject *kind_decode, *kind_prefill, *str_device;
 
@@ -72,8 +73,20 @@ bool stream_of(const Tensor& t, void*& stream) {
   return !PyErr_Occurred();
 }
 
-// The kept workspace of `kind` on t's device if it holds `bytes`; null: the wrapper allocates.
-void* workspace(const Tensor& t, PyObject* kind, size_t bytes) {
+// The workspace of a call on tensor t (of Python object o): the default stream's kept one if it holds
+// `bytes` (null: the wrapper allocates), on another stream that stream's, a reference to it in `ref`.
+struct Ref {
+  PyObject* o = nullptr;
+  ~Ref() { Py_XDECREF(o); }
+};
+void* workspace(PyObject* o, const Tensor& t, void* stream, PyObject* kind, size_t bytes, Ref& ref) {
+  if (stream != nullptr) {
+    PyObject* dev = PyObject_GetAttr(o, str_device);
+    ref.o = dev ? PyObject_CallFunction(side_workspace, "OnO", dev, (Py_ssize_t)bytes, kind) : nullptr;
+    Py_XDECREF(dev);
+    const Tensor* ws = ref.o ? plain(ref.o) : nullptr;
+    return ws ? ws->data_ptr() : nullptr;
+  }
   PyObject* idx = PyLong_FromLong(t.get_device());
   PyObject* key = idx ? PyTuple_Pack(2, idx, kind) : nullptr;
   PyObject* w = key ? PyDict_GetItemWithError(workspaces, key) : nullptr;
@@ -181,9 +194,12 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const size_t need = t.bs == 16 ? L.decode_ws(t.B, t.H, t.Hd, t.pages, t.split) : 0;
     Tensor records;  // the balanced launch: this call's own
     if (need && t.split < 0) records = at::empty({(int64_t)need}, t.q->options().dtype(at::kByte));
-    void* ws = !need ? nullptr : (t.split < 0 ? records.data_ptr() : workspace(*t.q, kind_decode, need));
     void* stream;
-    if ((need && ws == nullptr) || !stream_of(*t.q, stream)) return nullptr;
+    if (!stream_of(*t.q, stream)) return nullptr;
+    Ref held;
+    void* ws = !need ? nullptr
+                     : (t.split < 0 ? records.data_ptr() : workspace(a[0], *t.q, stream, kind_decode, need, held));
+    if (need && ws == nullptr) return nullptr;
     const Tensor& o = t.result();
     const void* ord = data(order);
     const int st = unlocked([&] {
@@ -204,10 +220,12 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Attn t;
     if (a[6] == Py_None || !t.parse(a, a[6], a[7])) return nullptr;
     const size_t need = t.bs == 16 ? L.prefill_ws(t.B, t.H, t.T, t.Hd, t.pages, t.split) : 0;
-    void* ws = need ? workspace(*t.q, kind_prefill, need) : nullptr;
     void* stream;
-    if ((need && ws == nullptr) || !stream_of(*t.q, stream)) return nullptr;
-    if (need && stream != nullptr) return nullptr;  // (the kept workspace is the default stream's)
+    if (!stream_of(*t.q, stream)) return nullptr;
+    if (need && stream != nullptr) return nullptr;  // (the wrapper's own)
+    Ref held;
+    void* ws = need ? workspace(a[0], *t.q, stream, kind_prefill, need, held) : nullptr;
+    if (need && ws == nullptr) return nullptr;
     const Tensor& o = t.result();
     const int st = unlocked([&] {
       return L.prefill(t.q->data_ptr(), t.q->stride(0), t.q->stride(1), t.q->stride(2), o.data_ptr(), o.stride(0),
@@ -313,10 +331,11 @@ PyObject* qkv_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// bind({name: address}, workspaces, raw stream lookup, check, default_split_blocks): the functions serve calls from here on.
+// bind({name: address}, workspaces, raw stream lookup, check, default_split_blocks, _call_workspace): the
+// functions serve calls from here on.
 PyObject* bind(PyObject*, PyObject* args) {
-  PyObject *addr, *ws, *rs, *ck, *sp;
-  if (!PyArg_ParseTuple(args, "O!O!OOO", &PyDict_Type, &addr, &PyDict_Type, &ws, &rs, &ck, &sp)) return nullptr;
+  PyObject *addr, *ws, *rs, *ck, *sp, *sw;
+  if (!PyArg_ParseTuple(args, "O!O!OOOO", &PyDict_Type, &addr, &PyDict_Type, &ws, &rs, &ck, &sp, &sw)) return nullptr;
   auto get = [&](const char* name, auto& fn) {
     PyObject* o = PyDict_GetItemString(addr, name);
     if (o == nullptr) {
@@ -331,11 +350,12 @@ PyObject* bind(PyObject*, PyObject* args) {
       !get("pa_prefill_workspace_size", L.prefill_ws) || !get("pa_kv_append", L.append) ||
       !get("pa_linear_rows", L.linear) || !get("pa_qkv_append", L.qkv))
     return nullptr;
-  Py_INCREF(ws); Py_INCREF(rs); Py_INCREF(ck); Py_INCREF(sp);
+  Py_INCREF(ws); Py_INCREF(rs); Py_INCREF(ck); Py_INCREF(sp); Py_INCREF(sw);
   Py_XSETREF(workspaces, ws);
   Py_XSETREF(raw_stream, rs);
   Py_XSETREF(fail, ck);
   Py_XSETREF(splits, sp);
+  Py_XSETREF(side_workspace, sw);
   ready = true;
   Py_RETURN_NONE;
 }

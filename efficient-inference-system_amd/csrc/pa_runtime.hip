@@ -2,7 +2,7 @@
 #include <stdarg.h>
 #include <string.h>
 
-#include "pa_common.h"
+#include "pa_attention.h"
 
 namespace pa_host {
 
@@ -32,6 +32,16 @@ int device_cu_count() {
 }
 
 }  // namespace pa_host
+
+extern "C" unsigned long long paged_internal_capture_id(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return status == hipStreamCaptureStatusNone ? 0 : id;
+}
 
 extern "C" int pa_version(void) { return 100; }  // 0.1.0
 

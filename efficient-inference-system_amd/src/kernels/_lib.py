@@ -146,6 +146,11 @@ SIGNATURES: dict[str, tuple] = {
     ),
 }
 
+# What the wrappers use beside the public entry points (declared in csrc/pa_attention.h).
+INTERNAL: dict[str, tuple] = {
+    "paged_internal_capture_id": (ctypes.c_uint64, [_c_void_p]),
+}
+
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 
@@ -167,7 +172,7 @@ def load() -> ctypes.CDLL:
                     "`python efficient-inference-system_amd/build_lib.py` (hipcc, gfx950)"
                 )
             lib = ctypes.CDLL(str(LIB_PATH))
-            for name, (restype, argtypes) in SIGNATURES.items():
+            for name, (restype, argtypes) in (SIGNATURES | INTERNAL).items():
                 fn = getattr(lib, name)
                 fn.restype = restype
                 fn.argtypes = argtypes

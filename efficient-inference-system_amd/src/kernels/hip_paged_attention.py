@@ -15,6 +15,7 @@ on a HIP device: there is no CPU path.
 from __future__ import annotations
 
 import math
+import threading
 
 import torch
 
@@ -27,6 +28,10 @@ except ImportError:  # not built: the Python versions run
 
 _workspaces: dict[tuple[int, str], torch.Tensor] = {}
 _retired_workspaces: list[torch.Tensor] = []
+# Workspaces off the default stream: (device, stream, kind) -> (capture, tensor), the latest used last.
+_stream_workspaces: dict[tuple[int, int, str], tuple[int, torch.Tensor]] = {}
+_stream_workspaces_lock = threading.Lock()
+MAX_STREAM_WORKSPACES = 8
 _cu_counts: dict[int, int] = {}
 
 
@@ -61,7 +66,7 @@ def cu_count(device: torch.device) -> int:
 
 
 def _workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
-    """The device's split-K workspace for `kind` ("decode" or "prefill"), at least `nbytes` long.
+    """The default stream's split-K workspace for `kind` ("decode" or "prefill"), at least `nbytes` long.
     Both kinds start with arrival counters of the in-launch merges, which must be zero before first
     use and stay zero between calls: workspaces are zero-filled when allocated, and the two kinds
     are kept apart (their layouts differ). A workspace replaced by a larger one stays allocated
@@ -73,6 +78,37 @@ def _workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
             _retired_workspaces.append(ws)
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _workspaces[(idx, kind)] = ws
+    return ws
+
+
+COUNTER_BYTES = {"decode": 256 << 10}  # PA_DECODE_COUNTER_BYTES in include/paged_hip.h
+
+
+def _capture_id(stream: int) -> int:
+    """Identifier of the graph capture that a stream (not the default one) is part of; 0: none."""
+    return _lib.load().paged_internal_capture_id(stream)
+
+
+def _call_workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
+    """The workspace of a call on `device`'s current stream: calls that follow each other on one stream
+    share one, calls on several streams and replays of several graphs never do (they would add to the
+    same arrival counters and overwrite each other's records). Under capture it comes from the graph's
+    memory, one per capture and stream, cleared by the first call that the graph replays. The stream
+    that allocated a workspace is the only one that uses it, so that one dropped here (at most
+    MAX_STREAM_WORKSPACES are held) is reused in stream order."""
+    stream = _stream_ptr(device)
+    if stream == 0:
+        return _workspace(device, nbytes, kind)
+    idx = device.index if device.index is not None else torch.cuda.current_device()
+    key, capture = (idx, stream, kind), _capture_id(stream)
+    with _stream_workspaces_lock:
+        held, ws = _stream_workspaces.pop(key, (0, None))
+        if ws is None or held != capture or ws.numel() < nbytes:
+            ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            ws[:COUNTER_BYTES[kind]].zero_()
+        _stream_workspaces[key] = (capture, ws)
+        while len(_stream_workspaces) > MAX_STREAM_WORKSPACES:
+            del _stream_workspaces[next(iter(_stream_workspaces))]
     return ws
 
 
@@ -143,7 +179,7 @@ def native_call():
             addresses = _lib.entry_addresses()
         except (RuntimeError, OSError):
             return None  # (the wrapper raises it once the call's own arguments are found good)
-        _call.bind(addresses, _workspaces, _raw_stream, _lib.check, default_split_blocks)
+        _call.bind(addresses, _workspaces, _raw_stream, _lib.check, default_split_blocks, _call_workspace)
         _call_bound = True
     return _call if _call_bound else None
 
@@ -205,6 +241,26 @@ def paged_attention_decode_hip(
         done = native.decode(q, k_pool, v_pool, page_table, seq_lens, current_lengths, order, split_blocks, out)
         if done is not None:
             return done
+    return decode_in_workspace(None, q, k_pool, v_pool, page_table, seq_lens, current_lengths, order=order,
+                               split_blocks=split_blocks, out=out)
+
+
+def decode_in_workspace(
+    ws: torch.Tensor | None,
+    q: torch.Tensor,
+    k_pool: torch.Tensor,
+    v_pool: torch.Tensor,
+    page_table: torch.Tensor,
+    seq_lens: torch.Tensor,
+    current_lengths: torch.Tensor,
+    *,
+    order: torch.Tensor | None = None,
+    split_blocks: int | None = None,
+    out: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """paged_attention_decode_hip on a workspace of the caller's (uint8, as long as
+    pa_decode_workspace_size says, its counters zero and no other call's meanwhile); None: the
+    stream's."""
     _require_gpu("paged_attention_decode_hip", q, k_pool, v_pool, page_table, seq_lens, current_lengths)
     _check_pool("paged_attention_decode_hip", k_pool, v_pool)
     B, H, T, Hd = q.shape
@@ -229,11 +285,12 @@ def paged_attention_decode_hip(
         split_blocks = default_split_blocks(B, H, max_pages, q.device, order is not None)
     lib = _lib.load()
     ws_bytes = lib.pa_decode_workspace_size(B, H, Hd, max_pages, split_blocks) if bs == 16 else 0
-    ws = None
-    if ws_bytes:  # (the balanced launch: records only, this call's own)
-        ws = _workspace(q.device, ws_bytes, "decode") if split_blocks > 0 else \
+    if ws_bytes and ws is None:  # (the balanced launch: records only, this call's own)
+        ws = _call_workspace(q.device, ws_bytes, "decode") if split_blocks > 0 else \
             torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    ws_ptr = ws.data_ptr() if ws is not None else None
+    elif ws_bytes and ws.numel() < ws_bytes:
+        raise ValueError(f"the workspace has {ws.numel()} bytes, the call needs {ws_bytes}")
+    ws_ptr = ws.data_ptr() if ws_bytes else None
     status = lib.pa_decode(
         q.data_ptr(), q.stride(0), q.stride(1),
         out.data_ptr(), out.stride(0), out.stride(1), _lib.dtype_code(q.dtype),

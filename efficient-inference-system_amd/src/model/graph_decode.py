@@ -62,8 +62,8 @@ import torch
 from src.cache.paged_kv import BatchedPagedKVCache, KVStorage
 from src.kernels import _lib, hip_linear
 from src.kernels.hip_paged_attention import (
-    _stream_ptr, _workspace, argmax_rows_hip, default_prefill_split_blocks, default_split_blocks, kv_append_hip,
-    pack_metadata_mirror_hip, paged_attention_decode_hip, paged_attention_prefill_hip)
+    _stream_ptr, argmax_rows_hip, decode_in_workspace, default_prefill_split_blocks, default_split_blocks,
+    kv_append_hip, pack_metadata_mirror_hip, paged_attention_prefill_hip)
 from src.kernels.staging import MappedHostWords
 
 try:  # native host bookkeeping (csrc/host/paged_host.cpp): same results as the Python below
@@ -328,11 +328,10 @@ class _Captured:
         else:
             self.split_blocks = default_prefill_split_blocks(B, H, Tb, pages, device, pools[0].dtype)
             ws_bytes = lib.pa_prefill_workspace_size(B, H, Tb, Hd, pages, self.split_blocks)
-        # Allocated outside the capture and referenced here, so the address the graph records
-        # stays valid for the graph's lifetime. (Prefill calls and a balanced decode take theirs from
-        # the graph's own pool.)
-        kept = ws_bytes and Tb == 1 and self.split_blocks > 0
-        self.ws = _workspace(device, ws_bytes, "decode") if kept else None
+        # The decode calls' workspace (one after another, layer by layer): this graph's own, so that
+        # replays of other graphs and eager calls, on whichever streams, never share it, and zeroed
+        # once, outside the capture, since every call leaves its counters zero.
+        self.ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes and Tb == 1 else None
         self.fused = B * Tb <= FUSED_STEP_ROWS and fused_decode_enabled() and hip_linear.model_supported(model)
         # Steps of at most 16 rows of an fp32 model (every decode step at batch <= 16): per layer
         # four launches, the MLP in one (fc1 column tiles adding their fc2 shares with atomic adds).
@@ -425,7 +424,7 @@ class GraphedStep:
             v_new = a.heads(a.v_proj(h))
             kv_append_hip(k_new, v_new, k_pool, v_pool, slots)
             if Tb == 1:
-                o = paged_attention_decode_hip(q, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
+                o = decode_in_workspace(cap.ws, q, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
             else:
                 o = paged_attention_prefill_hip(q, k_pool, v_pool, pt, seq32, cap.cur,
                                                 split_blocks=cap.split_blocks)
@@ -450,7 +449,7 @@ class GraphedStep:
             q = hip_linear.qkv_append_hip(x, blk.ln1, a, k_pool, v_pool, slots)
             q4 = q.view(B, Tb, a.num_heads, a.head_dim).transpose(1, 2)
             if Tb == 1:
-                o = paged_attention_decode_hip(q4, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
+                o = decode_in_workspace(cap.ws, q4, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
             else:
                 o = paged_attention_prefill_hip(q4, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
             o2 = o.transpose(1, 2).reshape(rows, a.d_model)
