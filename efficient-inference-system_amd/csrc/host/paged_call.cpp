@@ -52,6 +52,10 @@ bool optional(PyObject* o, const Tensor*& t) {
   return o == Py_None || (t = plain(o)) != nullptr;
 }
 bool on_gpu(const Tensor* t) { return t != nullptr && t->is_cuda(); }
+// An optional operand that a kernel reads: on the GPU, whole, of at least `entries` elements.
+bool readable(const Tensor* t, int64_t entries) {
+  return t == nullptr || (t->is_cuda() && t->is_contiguous() && t->numel() >= entries);
+}
 int dtype_of(const Tensor& t) {
   return t.scalar_type() == at::kFloat ? PA_DTYPE_F32 : (t.scalar_type() == at::kBFloat16 ? PA_DTYPE_BF16 : -1);
 }
@@ -153,6 +157,7 @@ struct Attn {
     nblk = k->size(0); bs = k->size(2);
     pages = pt->size(1); pt_stride = pt->stride(0);
     if (k->size(1) != H || k->size(3) != Hd || B == 0 || pages == 0) return false;
+    if (pt->size(0) < B || sl->numel() < B || cl->numel() < B) return false;
     if (!fits32(B) || !fits32(H) || !fits32(T) || !fits32(Hd) || !fits32(bs) || !fits32(pages)) return false;
     if (out != nullptr && (!out->is_cuda() || out->device() != q->device() || out->sizes() != q->sizes() ||
                            out->scalar_type() != q->scalar_type() || out->stride(3) != 1))
@@ -179,7 +184,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Attn t;
     const Tensor* order;
     if (!t.parse(a, a[7], a[8]) || t.T != 1 || !optional(a[6], order)) return nullptr;
-    if (order != nullptr && !(order->scalar_type() == at::kInt && order->is_contiguous())) return nullptr;
+    if (order != nullptr && !(order->scalar_type() == at::kInt && readable(order, t.B))) return nullptr;
     if (a[7] == Py_None) {
       PyObject* dev = PyObject_GetAttr(a[0], str_device);
       PyObject* sb = dev ? PyObject_CallFunction(splits, "LLLOO", (long long)t.B, (long long)t.H, (long long)t.pages,
@@ -267,6 +272,11 @@ bool rows2d(const Tensor* t, int dt) {
   return on_gpu(t) && t->dim() == 2 && t->stride(1) == 1 && dtype_of(*t) >= 0 && (dt < 0 || dtype_of(*t) == dt);
 }
 bool typed(const Tensor* t, int dt) { return t == nullptr || dtype_of(*t) == dt; }
+bool holds(const Tensor* t, int64_t rows, int64_t cols) { return t == nullptr || (t->size(0) >= rows && t->size(1) >= cols); }
+// A layer's parameters: weight [rows, cols], bias.
+bool parameters(const Tensor* w, const Tensor* b, int64_t rows, int64_t cols) {
+  return w->dim() == 2 && w->size(0) == rows && w->size(1) == cols && readable(w, rows * cols) && readable(b, rows);
+}
 
 // linear_rows(x, weight, bias, ln_weight, ln_bias, ln_eps, gelu, residual, out, copy_to)
 PyObject* linear_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -282,7 +292,8 @@ PyObject* linear_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return nullptr;
     const int64_t N = w->size(0);
     if ((res && !rows2d(res, dt)) || (out && !rows2d(out, dt)) || (cp && !rows2d(cp, dt))) return nullptr;
-    if (cp && (cp->size(0) < M || cp->size(1) < N)) return nullptr;
+    if (!parameters(w, b, N, K) || !readable(lw, K) || !readable(lb, K)) return nullptr;
+    if (!holds(res, M, N) || !holds(out, M, N) || !holds(cp, M, N)) return nullptr;
     if (!fits32(M) || !fits32(K) || !fits32(N)) return nullptr;
     const double eps = PyFloat_AsDouble(a[5]);
     const int gelu = PyObject_IsTrue(a[6]);
@@ -312,8 +323,11 @@ PyObject* qkv_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
       if (w[i] == nullptr || !optional(a[5 + 2 * i], b[i]) || !typed(w[i], dt) || !typed(b[i], dt)) return nullptr;
     }
     const int64_t M = x->size(0), D = x->size(1);
-    if ((out && !rows2d(out, dt)) || !pools(k, v) || sm == nullptr || sm->scalar_type() != at::kInt ||
-        sm->numel() < M || !sm->is_contiguous() || !fits32(M) || !fits32(D) || !fits32(k->size(1)) ||
+    for (int i = 0; i < 3; ++i)
+      if (!parameters(w[i], b[i], D, D)) return nullptr;
+    if (!readable(lw, D) || !readable(lb, D)) return nullptr;
+    if ((out && (!rows2d(out, dt) || !holds(out, M, D))) || !pools(k, v) || sm == nullptr || sm->scalar_type() != at::kInt ||
+        !readable(sm, M) || !fits32(M) || !fits32(D) || !fits32(k->size(1)) ||
         !fits32(k->size(2)) || !fits32(k->size(3)))
       return nullptr;
     const double eps = PyFloat_AsDouble(a[3]);

@@ -21,7 +21,7 @@ import torch
 import torch.nn as nn
 
 from src.kernels import _lib
-from src.kernels.hip_paged_attention import _stream_ptr, native_call
+from src.kernels.hip_paged_attention import _require_readable, _stream_ptr, native_call
 
 MAX_ROWS = 2048  # rows per call accepted by the library
 SUPPORTED_FEATURES = (128, 256, 512, 1024, 2048)
@@ -52,6 +52,32 @@ def _same_dtype(dtype: torch.dtype, *tensors) -> None:
             raise ValueError(f"all operands must be {dtype}, got a {t.dtype} tensor")
 
 
+def _holds(name: str, t: torch.Tensor | None, rows: int, cols: int) -> None:
+    if t is not None and (t.shape[0] < rows or t.shape[1] < cols):
+        raise ValueError(f"{name} must hold {rows} rows of {cols} features, got {tuple(t.shape)}")
+
+
+def _parameters(linear: nn.Linear, rows: int, cols: int) -> None:
+    """A layer's parameters as the kernels read them: [rows, cols] and [rows], contiguous, in memory that
+    they reach."""
+    if tuple(linear.weight.shape) != (rows, cols) or not linear.weight.is_contiguous():
+        raise ValueError(f"the weight must be contiguous [{rows}, {cols}], got {tuple(linear.weight.shape)}")
+    _require_readable("weight", linear.weight)
+    _vector("bias", linear.bias, rows)
+
+
+def _vector(name: str, t: torch.Tensor | None, entries: int) -> None:
+    _require_readable(name, t, entries)
+    if t is not None and not t.is_contiguous():
+        raise ValueError(f"{name} must be contiguous")
+
+
+def _norm(ln: nn.LayerNorm | None, features: int) -> None:
+    if ln is not None:
+        _vector("LayerNorm weight", ln.weight, features)
+        _vector("LayerNorm bias", ln.bias, features)
+
+
 def supported(linear: nn.Linear) -> bool:
     return (linear.weight.dtype in DTYPES and linear.weight.is_contiguous()
             and (linear.bias is None or linear.bias.dtype == linear.weight.dtype)
@@ -78,15 +104,14 @@ def linear_rows_hip(x: torch.Tensor, linear: nn.Linear, *, ln: nn.LayerNorm | No
     _same_dtype(dt, linear.weight, linear.bias, ln.weight if ln is not None else None,
                 ln.bias if ln is not None else None)
     N = linear.out_features
+    _parameters(linear, N, K)
+    _norm(ln, K)
     if out is None:
         out = torch.empty((M, N), dtype=dt, device=x.device)
-    _rows(out, "out", dt)
-    if residual is not None:
-        _rows(residual, "residual", dt)
-    if copy_to is not None:
-        _rows(copy_to, "copy_to", dt)
-        if copy_to.shape[0] < M or copy_to.shape[1] < N:
-            raise ValueError(f"copy_to must hold {M} rows of {N} features")
+    for name, t in (("out", out), ("residual", residual), ("copy_to", copy_to)):
+        if t is not None:
+            _rows(t, name, dt)
+            _holds(name, t, M, N)
     status = _lib.load().pa_linear_rows(
         x.data_ptr(), x.stride(0), M, K,
         linear.weight.data_ptr(), _ptr(linear.bias), N,
@@ -126,6 +151,8 @@ def linear_select_rows_hip(x: torch.Tensor, group_rows: int, row_index: torch.Te
     _same_dtype(dt, linear.weight, linear.bias, ln.weight if ln is not None else None,
                 ln.bias if ln is not None else None)
     N = linear.out_features
+    _parameters(linear, N, K)
+    _norm(ln, K)
     if out is None:
         out = torch.empty((groups, N), dtype=dt, device=x.device)
     _rows(out, "out", dt)
@@ -174,9 +201,15 @@ def qkv_append_hip(x: torch.Tensor, ln: nn.LayerNorm, attn, k_pool: torch.Tensor
     M, D = x.shape
     _same_dtype(dt, ln.weight if ln is not None else None, ln.bias if ln is not None else None,
                 *(t for l in (attn.q_proj, attn.k_proj, attn.v_proj) for t in (l.weight, l.bias)))
+    for linear in (attn.q_proj, attn.k_proj, attn.v_proj):
+        _parameters(linear, D, D)
+    _norm(ln, D)
     if out is None:
         out = torch.empty((M, D), dtype=dt, device=x.device)
     _rows(out, "out", dt)
+    _holds("out", out, M, D)
+    for name, t in (("slot_mapping", slot_mapping), ("k_pool", k_pool), ("v_pool", v_pool)):
+        _require_readable(name, t)
     nblk, H, bs, Hd = k_pool.shape
     if slot_mapping.dtype != torch.int32 or slot_mapping.numel() < M or not slot_mapping.is_contiguous():
         raise ValueError("slot_mapping must be a contiguous int32 tensor with one entry per row")
@@ -209,9 +242,13 @@ def embed_rows_hip(ids: torch.Tensor, pos_start: torch.Tensor, token_emb: nn.Emb
             raise ValueError(f"{name} weight must be a contiguous float32 or bfloat16 table (both of one dtype)")
     B, T = ids.shape
     d = token_emb.embedding_dim
+    for name, t in (("ids", ids), ("pos_start", pos_start), ("token_emb weight", token_emb.weight),
+                    ("pos_emb weight", pos_emb.weight)):
+        _require_readable(name, t)
     if out is None:
         out = torch.empty((B * T, d), dtype=dt, device=ids.device)
     _rows(out, "out", dt)
+    _holds("out", out, B * T, d)
     status = _lib.load().pa_embed_rows(
         ids.data_ptr(), pos_start.data_ptr(), B, T, token_emb.weight.data_ptr(), token_emb.num_embeddings,
         pos_emb.weight.data_ptr(), pos_emb.num_embeddings, d, out.data_ptr(), out.stride(0), _lib.dtype_code(dt),
@@ -249,8 +286,12 @@ def mlp_rows_hip(x: torch.Tensor, ln: nn.LayerNorm, fc1: nn.Linear, fc2: nn.Line
     _rows(out, "out", torch.float32)
     if out.shape[0] < M or out.shape[1] != D:
         raise ValueError(f"out must hold {M} rows of {D} features")
+    _parameters(fc1, fc1.out_features, D)
+    _parameters(fc2, D, fc1.out_features)
+    _norm(ln, D)
     if residual is not None:
         _rows(residual, "residual", torch.float32)
+        _holds("residual", residual, M, D)
     status = _lib.load().pa_mlp_rows(
         x.data_ptr(), x.stride(0), M, D, ln.weight.data_ptr(), ln.bias.data_ptr(), float(ln.eps),
         fc1.weight.data_ptr(), _ptr(fc1.bias), fc1.out_features, 1 if gelu else 0,

@@ -53,6 +53,24 @@ def _require_gpu(name: str, *tensors: torch.Tensor) -> None:
             raise ValueError(f"{name}: the hip_paged backend needs tensors on a HIP device, got {t.device}")
 
 
+def _require_readable(name: str, t: torch.Tensor | None, entries: int = 0) -> None:
+    """A kernel reads t (None: nothing): device memory, or pinned host memory, of at least `entries`
+    elements."""
+    if t is None:
+        return
+    if not (t.is_cuda or t.is_pinned()):
+        raise ValueError(f"{name} must be on a HIP device, got {t.device}")
+    if t.numel() < entries:
+        raise ValueError(f"{name} has {t.numel()} entries, the call reads {entries}")
+
+
+def _require_requests(page_table: torch.Tensor, seq_lens: torch.Tensor, current_lengths: torch.Tensor, batch: int) -> None:
+    if page_table.dim() == 2 and page_table.shape[1] > 0 and page_table.shape[0] < batch:
+        raise ValueError(f"page_table has {page_table.shape[0]} rows for {batch} requests")
+    _require_readable("seq_lens", seq_lens, batch)
+    _require_readable("current_lengths", current_lengths, batch)
+
+
 def _require_i32(name: str, t: torch.Tensor) -> None:
     if t.dtype != torch.int32 or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous int32 tensor (got {t.dtype}, contiguous={t.is_contiguous()})")
@@ -274,8 +292,10 @@ def decode_in_workspace(
     _require_i32("page_table", page_table)
     _require_i32("seq_lens", seq_lens)
     _require_i32("current_lengths", current_lengths)
+    _require_requests(page_table, seq_lens, current_lengths, B)
     if order is not None:
         _require_i32("order", order)
+        _require_readable("order", order, B)
     if out is None:
         out = torch.empty_like(q)
     _check_out("paged_attention_decode_hip", out, q)
@@ -336,6 +356,7 @@ def paged_attention_prefill_hip(
     _require_i32("page_table", page_table)
     _require_i32("seq_lens", seq_lens)
     _require_i32("current_lengths", current_lengths)
+    _require_requests(page_table, seq_lens, current_lengths, B)
     if out is None:
         out = torch.empty_like(q)
     _check_out("paged_attention_prefill_hip", out, q)

@@ -96,3 +96,75 @@ def test_forms_left_to_the_wrapper(device):
         hpa.paged_attention_decode_hip(q, k, v, table.long(), lens, cur)
     with pytest.raises(RuntimeError):  # no data pointer under vmap: refused as by the wrapper
         torch.vmap(lambda y: hpa.paged_attention_decode_hip(y, k, v, table, lens, cur))(q[None])
+
+
+def _refused(call, *args, **kw):
+    with pytest.raises(ValueError):
+        call(*args, **kw)
+
+
+@pytest.mark.gpu
+def test_attention_operands_that_a_kernel_cannot_read(device):
+    """Host memory and arrays shorter than the batch are refused before any launch, by either front."""
+    for T, call in ((1, hpa.paged_attention_decode_hip), (16, hpa.paged_attention_prefill_hip)):
+        q, k, v, table, lens, cur = _attention(device, T)
+        want = call(q, k, v, table, lens, cur)
+        for bad in ((table[:2], lens, cur), (table, lens[:2], cur), (table, lens, cur[:2]), (table, lens, cur.cpu())):
+            _refused(call, q, k, v, *bad)
+        assert torch.equal(call(q, k, v, torch.cat([table, table]), torch.cat([lens, lens]), torch.cat([cur, cur])), want)
+    q, k, v, table, lens, cur = _attention(device, 1)
+    want = hpa.paged_attention_decode_hip(q, k, v, table, lens, cur)
+    order = torch.tensor([2, 0, 1], dtype=torch.int32)
+    for bad in (order, order[:2].to(device), order.long().to(device)):
+        _refused(hpa.paged_attention_decode_hip, q, k, v, table, lens, cur, order=bad)
+    for good in (order.to(device), order.pin_memory()):  # (kernels read pinned host memory in place)
+        assert torch.equal(hpa.paged_attention_decode_hip(q, k, v, table, lens, cur, order=good), want)
+    _refused(hpa.kv_append_hip, q, q, k, v, order)
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_layer_operands_that_a_kernel_cannot_reach(device):
+    M, K, N = 5, 128, 64
+    x = torch.randn(M, K, device=device)
+    lin, ln = nn.Linear(K, N).to(device), nn.LayerNorm(K).to(device)
+    rows = lambda m, n: torch.zeros(m, n, device=device)  # noqa: E731
+    call = hip_linear.linear_rows_hip
+    want = call(x, lin, ln=ln)
+    for name in ("out", "residual", "copy_to"):
+        for bad in (rows(M - 1, N), rows(M, N - 1), torch.zeros(M, N)):
+            _refused(call, x, lin, ln=ln, **{name: bad})
+    assert torch.equal(call(x, lin, ln=ln, out=rows(M + 1, N + 4))[:M, :N], want)
+    _refused(call, x, nn.Linear(K, N))
+    _refused(call, x, lin, ln=nn.LayerNorm(K))
+    _refused(call, x, lin, ln=nn.LayerNorm(K // 2).to(device))
+    strided = nn.Linear(K, N).to(device)
+    strided.weight = nn.Parameter(torch.randn(K, N, device=device).t())
+    _refused(call, x, strided)
+    short = nn.Linear(K, N).to(device)
+    short.bias = nn.Parameter(torch.zeros(N - 1, device=device))
+    _refused(call, x, short)
+    index = torch.zeros(1, dtype=torch.int32, device=device)
+    _refused(hip_linear.linear_select_rows_hip, x, M, index, nn.Linear(K, N))
+
+    layers = {n: nn.Linear(K, K).to(device) for n in ("q_proj", "k_proj", "v_proj")}
+    attn = lambda **kw: type("A", (), {**layers, **kw})()  # noqa: E731
+    pools = [torch.zeros(4, 2, 16, 64, device=device) for _ in range(2)]
+    slots = torch.arange(M, dtype=torch.int32)
+    qkv = hip_linear.qkv_append_hip
+    qkv(x, ln, attn(), *pools, slots.to(device))
+    _refused(qkv, x, ln, attn(), *pools, slots)
+    _refused(qkv, x, ln, attn(), *pools, slots[: M - 1].to(device))
+    _refused(qkv, x, ln, attn(), *pools, slots.to(device), out=rows(M - 1, K))
+    _refused(qkv, x, ln, attn(k_proj=nn.Linear(K, K)), *pools, slots.to(device))
+    _refused(qkv, x, ln, attn(v_proj=nn.Linear(K, K // 2).to(device)), *pools, slots.to(device))
+    _refused(qkv, x, ln, attn(), *(p.cpu() for p in pools), slots.to(device))
+
+    fc1, fc2 = nn.Linear(K, N).to(device), nn.Linear(N, K).to(device)
+    _refused(hip_linear.mlp_rows_hip, x, ln, fc1, nn.Linear(N, K), rows(M, K))
+    _refused(hip_linear.mlp_rows_hip, x, ln, fc1, fc2, rows(M, K), residual=rows(M - 1, K))
+    ids, pos = torch.zeros(2, 3, dtype=torch.int64), torch.zeros(2, dtype=torch.int64)
+    table = nn.Embedding(8, K).to(device)
+    _refused(hip_linear.embed_rows_hip, ids.to(device), pos, table, table)
+    _refused(hip_linear.embed_rows_hip, ids.to(device), pos.to(device), nn.Embedding(8, K), table)
+    _refused(hip_linear.embed_rows_hip, ids.to(device), pos.to(device), table, table, out=rows(5, K))
