@@ -77,7 +77,7 @@ T_BUCKETS = (16, 32, 64, 96, 128, 160, 192, 224, 256)
 
 # Largest step (rows = B * bucketed T) for which each fused launch beats torch's layers, per
 # dtype. Measured in HIP-graph replay on MI355X (fused vs torch, us), d_model 512, d_ff 2048,
-# vocab 5000, with the library's choice between its 16-row and tiled kernels:
+# vocab 5000, with the library's choice between its 16-row, tiled and (LayerNorm, 512 features) block kernels:
 #   LayerNorm + q/k/v + append  fp32 11.8 at 256 rows, 22.9 vs 40.4 at 1024 (torch without the
 #                               append); bf16 13.5 vs 33.4 at 1024
 #   out_proj + residual         fp32 8.6 vs 11.0 at 1024, 12.6 vs 13.0 at 1536; bf16 5.0 vs 8.0 at 1024
@@ -92,6 +92,15 @@ FUSED_ROWS = {
     torch.bfloat16: {"qkv": 1024, "out_proj": 1024, "fc1": 1024, "fc2": 1024, "lm_head": 64},
 }
 FUSED_STEP_ROWS = 1024  # steps above this run the torch layers throughout
+# fc1 of models wider than 512. The limits above rest on the block kernel, which serves 512 features; fewer
+# stay ahead on the tiled kernel (256 features, d_ff 1024, 1024 rows, fused vs torch, us: fp32 13.6 vs 16.3,
+# bf16 8.4 vs 13.0), more fall behind it the more rows there are (1024 features, d_ff 4096: fp32 84 vs 46 at
+# 512 rows, 124 vs 66 at 768, 165 vs 81 at 1024; bf16 33 vs 20 at 512, 61 vs 27 at 1024).
+WIDE_FC1_ROWS = {torch.float32: 768, torch.bfloat16: 512}
+
+
+def fc1_row_limit(dtype: torch.dtype, d_model: int) -> int:
+    return FUSED_ROWS[dtype]["fc1"] if d_model <= 512 else WIDE_FC1_ROWS[dtype]
 
 
 def graphs_enabled() -> bool:
@@ -439,7 +448,7 @@ class GraphedStep:
         B, Tb = cap.B, cap.Tb
         lim = FUSED_ROWS[x.dtype]
         rows = B * Tb
-        fc1_fused, fc2_fused = rows <= lim["fc1"], rows <= lim["fc2"]
+        fc1_fused, fc2_fused = rows <= fc1_row_limit(x.dtype, x.shape[1]), rows <= lim["fc2"]
         # Folded MLP: x stays the residual buffer; out_proj writes x1 into x1_buf (the MLP's input)
         # and into x itself, and the MLP launch adds fc2's output (fc1 tile by fc1 tile) to x.
         x1_buf = torch.empty_like(x) if cap.folded else None
