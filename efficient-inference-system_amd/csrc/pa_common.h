@@ -39,8 +39,12 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 
 // fp32 products on the bf16 matrix cores: an fp32 operand as the sum of three bf16 parts, a product
 // as the six partial products of parts whose indices add up to at most 4. Values from kSplitMax on
-// (infinities among them) have no such split whose products stay finite.
+// (infinities among them) have no such split whose products stay finite. Small values lose bits: a
+// part is whole only where the value's last bit is a normal bf16, i.e. from about 2^-103 on. Operands
+// whose relative error counts are therefore split as kSplitScale times themselves, which brings the
+// last bit of every fp32 value (2^-149 at least) there, and the sums divided by the same.
 constexpr float kSplitMax = 1152921504606846976.f;  // 2^60
+constexpr float kSplitScale = 16777216.f;           // 2^24
 
 // Two fp32 values as packed bf16 triples: x = w1 + w2 + w3, each part the nearest bf16 of the rest.
 __device__ __forceinline__ void split_bf16x3(float lo, float hi, uint32_t& w1, uint32_t& w2, uint32_t& w3) {

@@ -787,9 +787,11 @@ __global__ __launch_bounds__(kTileWaves * kWave) void tile_linear_kernel(const L
 //   fp32: every operand is the sum of three bf16 parts and every product its six leading partial
 //   products (split_bf16x3), the leading one accumulated apart from the others (error 1.7e-7 of the
 //   norm at K 512, fp32 MFMA 2.4e-7). The fp32 MFMA runs at 1/16 of the bf16 rate and bounded the
-//   tiled kernel; six bf16 products take 6/16 of its time. Values of 2^60 and more (infinities among
-//   them) have no split with finite products: a workgroup that meets one forms its tile again with
-//   v_mfma_f32_32x32x2_f32 on operands from memory.
+//   tiled kernel; six bf16 products take 6/16 of its time. Both operands are split as kSplitScale
+//   times themselves, so that the split of every fp32 value is exact (weights of 2^-120: error 1.4e-3
+//   of the norm without). Values of 2^34 and more (infinities among them) then have no split with
+//   finite products: a workgroup that meets one forms its tile again with v_mfma_f32_32x32x2_f32 on
+//   operands from memory.
 //   bf16: one plane, the operands as they are.
 //   bound: LDS, which serves each wavefront 6 KB per six MFMAs (its peak), and the latency of a
 //   chunk: 1.6k cycles of which the MFMAs take 768.
@@ -803,6 +805,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kBlockK = 512;  // features
+constexpr float kBlockSplitMax = 17179869184.f;  // 2^34: 512 products of two such, times kSplitScale^2, are finite
 constexpr int kBlockRows = 128, kBlockCols = 64;
 
 template <typename T>
@@ -950,6 +953,8 @@ void block_linear_kernel(const LinArgs a) {
         }
         mx = fmaxf(fmaxf(mx, fabsf(f[0])), fabsf(f[1]));
         mx = fmaxf(fmaxf(mx, fabsf(f[2])), fabsf(f[3]));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] *= kSplitScale;
         uint32_t lo[3], hi[3];
         split_bf16x3(f[0], f[1], lo[0], lo[1], lo[2]);
         split_bf16x3(f[2], f[3], hi[0], hi[1], hi[2]);
@@ -1022,8 +1027,8 @@ void block_linear_kernel(const LinArgs a) {
   static_assert(nch % D == 0, "whole rounds of the ring");
   for (int ch0 = 0; ch0 < nch; ch0 += D) static_for<0, D>([&](auto dc) { iteration(dc, ch0 + decltype(dc)::value); });
   if constexpr (!BF) {
-    if (mx >= kSplitMax) sm_bad = 1;
-    acc += rest;
+    if (mx >= kBlockSplitMax) sm_bad = 1;
+    acc = (acc + rest) * (1.f / (kSplitScale * kSplitScale));
   }
   __syncthreads();  // stages are free; sm_bad is published
   if constexpr (!BF) {

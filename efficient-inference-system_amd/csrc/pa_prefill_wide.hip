@@ -722,10 +722,10 @@ void prefill_wide_kernel(const AttnArgs a) {
 }
 
 // fp32 KV: the bf16 kernel's workgroup layout, operand layouts and online softmax, with every fp32
-// operand as the sum of three bf16 parts (split_bf16x3: 8 + 8 + 8 significant bits, exact to
-// 2^-26 of the value) and every fp32 product as the six partial products whose parts' indices add
-// up to at most 4, on v_mfma_f32_32x32x16_bf16 with fp32 accumulation. The dropped partial products
-// are below 2^-25 of the product, i.e. below fp32's own rounding of it.
+// operand as the sum of three bf16 parts (split_bf16x3: 8 + 8 + 8 significant bits, fp32's 24) and every
+// fp32 product as the six partial products whose parts' indices add up to at most 4, on
+// v_mfma_f32_32x32x16_bf16 with fp32 accumulation. The dropped partial products are below 2^-25 of the
+// product, i.e. below fp32's own rounding of it.
 //   bound: the matrix cores. The fp32 MFMA (32x32x2) runs at 1/16 of the bf16 rate, so six bf16
 //   products take 6/16 of its time; a 32-key step at head_dim 128 is 96 bf16 MFMAs of 32 cycles
 //   against 128 fp32 ones of 64. K and V are split once per workgroup (not once per wavefront) on
@@ -743,6 +743,10 @@ void prefill_wide_kernel(const AttnArgs a) {
 // wavefront whose q or whose workgroup's K or V held one walks its steps a second time, with
 // v_mfma_f32_32x32x2_f32 on operands read straight from memory (slow; fp32 products as they are).
 // NaN needs no care: its parts are NaN.
+// V is split as kSplitScale times itself, so that the split of every fp32 value is exact (V of N(0, 1) *
+// 2^-120: error 3.5e-5 of the norm without, 2e-7 with it). K and q need no scale: where a part of one falls
+// short, the other is below 2^60 and the score off by less than 2^-50, as nothing to its exponential; and
+// weights below 2^-103 are to their row's largest, which is at least 1, what fp32's rounding of it is.
 template <typename IO, int HD, bool BAL>
 __global__ __launch_bounds__(kWideWaves * kWave) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_wide_f32_kernel(const AttnArgs a) {
@@ -958,14 +962,14 @@ void prefill_wide_f32_kernel(const AttnArgs a) {
   ++piece;
   auto lstore = [&]() {
     float mx = 0.f;
-    auto put = [&](const f32x4 (&x)[2], uint16_t* dst) {
+    auto put = [&](const f32x4 (&x)[2], uint16_t* dst, float scale) {
       u32x4 w1, w2, w3;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float lo = x[e >> 1][2 * (e & 1)], hi = x[e >> 1][2 * (e & 1) + 1];
         mx = fmaxf(fmaxf(mx, fabsf(lo)), fabsf(hi));
         uint32_t p1, p2, p3;
-        split_bf16x3(lo, hi, p1, p2, p3);
+        split_bf16x3(lo * scale, hi * scale, p1, p2, p3);
         w1[e] = p1; w2[e] = p2; w3[e] = p3;
       }
       *reinterpret_cast<u32x4*>(dst) = w1;
@@ -976,8 +980,8 @@ void prefill_wide_f32_kernel(const AttnArgs a) {
     for (int n = 0; n < CPT; ++n) {
       const int q = threadIdx.x + n * NW * kWave;
       const int kk = q / CPR, p = q % CPR;
-      put(kr[n], sbuf + kk * HD + 8 * (p ^ kswz(kk)));
-      put(vr[n], sbuf + 3 * PLANE + kk * HD + 8 * (p ^ vswz(kk)));
+      put(kr[n], sbuf + kk * HD + 8 * (p ^ kswz(kk)), 1.f);
+      put(vr[n], sbuf + 3 * PLANE + kk * HD + 8 * (p ^ vswz(kk)), kSplitScale);
     }
     if (mx >= kSplitMax) sm_bad = piece;
   };
@@ -1157,6 +1161,9 @@ void prefill_wide_f32_kernel(const AttnArgs a) {
               oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vp[32 * d], sacc[4 * j + r], oacc[d], 0, 0, 0);
           }
       }
+    } else {
+#pragma unroll
+      for (int d = 0; d < DU; ++d) oacc[d] *= 1.f / kSplitScale;
     }
   }
 

@@ -106,3 +106,22 @@ def test_default_choice_near_its_line(device, monkeypatch, rows):
     x = torch.randn(rows, K, device=device)
     want = F.gelu(_want(x, lin, ln))
     assert float((linear_rows_hip(x, lin, ln=ln, gelu=True).double() - want).norm() / want.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("where", ["weight", "norm"])
+@pytest.mark.parametrize("exponent", [-20, -90, -112, -120, -126, -136])
+@torch.no_grad()
+def test_small_values_keep_their_bits(device, monkeypatch, where, exponent):
+    """Weights, or normalised rows, down to fp32's denormals, whose bf16 parts would be no normal numbers."""
+    monkeypatch.setenv("PAGED_HIP_LINEAR_KERNEL", "block")
+    lin, ln = _layer(130, torch.float32, device, -exponent, bias=False)
+    x = torch.randn(150, K, device=device)
+    if where == "weight":
+        lin.weight.mul_(2.0**exponent)
+    else:
+        ln.weight.mul_(2.0**exponent)
+        ln.bias.mul_(2.0**exponent)
+    want = _want(x, lin, ln)
+    # (the normalised rows are rounded to fp32, at denormal scales to their spacing, and so is the result)
+    small = 2.0**-149 * (want.numel() ** 0.5) * (1 if where == "weight" else (1 + float(lin.weight.norm(dim=1).max())))
+    assert float((linear_rows_hip(x, lin, ln=ln).double() - want).norm()) < 1e-6 * float(want.norm()) + small

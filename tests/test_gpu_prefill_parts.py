@@ -92,3 +92,17 @@ def test_scales_far_from_one(device, monkeypatch, scale):
     case = (q / scale, k * scale, v * scale, table, lens, cur)
     got, ref = _run(case, device, monkeypatch, "wide"), _run(case, device, monkeypatch, "tile")
     assert float((got - ref).abs().max()) < 1e-5 * scale
+
+
+@pytest.mark.parametrize("balance", ["off", "force"])
+@pytest.mark.parametrize("Hd", [64, 128])
+@pytest.mark.parametrize("exponent", [-100, -112, -120, -126, -136, -147])
+def test_small_values_keep_their_bits(device, monkeypatch, exponent, Hd, balance):
+    """V down to fp32's denormals, whose bf16 parts would be no normal numbers."""
+    q, k, v, table, lens, cur = _case(Hd, [150, 700], 140, Hd - exponent)
+    case = (q, k, v * 2.0**exponent, table, lens, cur)
+    want = _f64(case)
+    got = _run(case, device, monkeypatch, "wide", balance).double()
+    # as test_error_of_fp32_sums, and two roundings to the denormals' spacing
+    bound = 2.0**-24 * (4 + (12 * max(lens) / 32) ** 0.5) * float(want.norm()) + 2.0**-149 * want.numel() ** 0.5
+    assert float((got - want).norm()) <= bound
