@@ -104,7 +104,7 @@ def build_call(verbose: bool = False) -> Path:
     _run([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
           f"-I{sysconfig.get_paths()['include']}", f"-isystem{tdir / 'include'}",
-          f"-isystem{tdir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{INCLUDE}", str(CALL_SRC),
+          f"-isystem{tdir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{INCLUDE}", f"-I{CSRC}", str(CALL_SRC),
           f"-L{tdir / 'lib'}", f"-Wl,-rpath,{tdir / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
           "-o", str(out) + ".tmp"], verbose)
     os.replace(str(out) + ".tmp", out)

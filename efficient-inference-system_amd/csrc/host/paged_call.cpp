@@ -20,6 +20,7 @@
 #include <cmath>
 
 #include "paged_hip.h"
+#include "pa_internal.h"
 
 namespace {
 
@@ -27,7 +28,7 @@ struct Lib {
   decltype(&pa_decode) decode = nullptr;
   decltype(&pa_decode_workspace_size) decode_ws = nullptr;
   decltype(&pa_prefill) prefill = nullptr;
-  decltype(&pa_prefill_workspace_size) prefill_ws = nullptr;
+  decltype(&paged_internal_prefill_workspace) prefill_ws = nullptr;
   decltype(&pa_kv_append) append = nullptr;
   decltype(&pa_linear_rows) linear = nullptr;
   decltype(&pa_qkv_append) qkv = nullptr;
@@ -224,10 +225,9 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     Attn t;
     if (a[6] == Py_None || !t.parse(a, a[6], a[7])) return nullptr;
-    const size_t need = t.bs == 16 ? L.prefill_ws(t.B, t.H, t.T, t.Hd, t.pages, t.split) : 0;
+    const size_t need = t.bs == 16 ? L.prefill_ws(dtype_of(*t.k), t.B, t.H, t.T, t.Hd, t.pages, t.split) : 0;
     void* stream;
     if (!stream_of(*t.q, stream)) return nullptr;
-    if (need && stream != nullptr) return nullptr;  // (the wrapper's own)
     Ref held;
     void* ws = need ? workspace(a[0], *t.q, stream, kind_prefill, need, held) : nullptr;
     if (need && ws == nullptr) return nullptr;
@@ -361,7 +361,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   };
   if (!get("pa_decode", L.decode) || !get("pa_decode_workspace_size", L.decode_ws) ||
       !get("pa_prefill", L.prefill) ||
-      !get("pa_prefill_workspace_size", L.prefill_ws) || !get("pa_kv_append", L.append) ||
+      !get("paged_internal_prefill_workspace", L.prefill_ws) || !get("pa_kv_append", L.append) ||
       !get("pa_linear_rows", L.linear) || !get("pa_qkv_append", L.qkv))
     return nullptr;
   Py_INCREF(ws); Py_INCREF(rs); Py_INCREF(ck); Py_INCREF(sp); Py_INCREF(sw);

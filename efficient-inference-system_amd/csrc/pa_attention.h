@@ -80,7 +80,3 @@ int launch_prefill_split(const AttnArgs& a, int io_dtype, hipStream_t stream);
 int launch_generic_attention(const AttnArgs& a, int io_dtype, int kv_dtype, hipStream_t stream);
 
 }  // namespace pa
-
-// For this package's own wrappers, beside the public entry points.
-// Identifier of the graph capture that `stream` (not the default stream) is part of; 0: none.
-extern "C" unsigned long long paged_internal_capture_id(void* stream);

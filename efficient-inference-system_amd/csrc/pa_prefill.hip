@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "pa_attention.h"
+#include "pa_internal.h"
 
 namespace pa {
 
@@ -718,11 +719,18 @@ using namespace pa;
 
 extern "C" size_t pa_prefill_workspace_size(int32_t batch, int32_t num_heads, int32_t query_len, int32_t head_dim,
                                             int32_t max_pages, int32_t split_blocks) {
+  const size_t b = paged_internal_prefill_workspace(PA_DTYPE_BF16, batch, num_heads, query_len, head_dim, max_pages,
+                                                    split_blocks);
+  const size_t f = paged_internal_prefill_workspace(PA_DTYPE_F32, batch, num_heads, query_len, head_dim, max_pages,
+                                                    split_blocks);
+  return b > f ? b : f;
+}
+
+extern "C" size_t paged_internal_prefill_workspace(int kv_dtype, int32_t batch, int32_t num_heads, int32_t query_len,
+                                                   int32_t head_dim, int32_t max_pages, int32_t split_blocks) {
   if (batch <= 0 || num_heads <= 0 || query_len <= 0 || !prefill_fast_shape(head_dim, 16)) return 0;
-  if (split_blocks < 0) {  // the larger of the bf16 and fp32 KV launches' needs
-    const int64_t gb = prefill_balanced_grid(batch, num_heads, query_len, head_dim, max_pages, PA_DTYPE_BF16);
-    const int64_t gf = prefill_balanced_grid(batch, num_heads, query_len, head_dim, max_pages, PA_DTYPE_F32);
-    const int64_t grid = gb > gf ? gb : gf;
+  if (split_blocks < 0) {
+    const int64_t grid = prefill_balanced_grid(batch, num_heads, query_len, head_dim, max_pages, kv_dtype);
     return grid > 0 ? PA_PREFILL_COUNTER_BYTES + prefill_balanced_record_bytes(grid, head_dim) : 0;
   }
   const int s = prefill_num_splits(max_pages, split_blocks);

@@ -2,7 +2,8 @@
 #include <stdarg.h>
 #include <string.h>
 
-#include "pa_attention.h"
+#include "pa_common.h"
+#include "pa_internal.h"
 
 namespace pa_host {
 

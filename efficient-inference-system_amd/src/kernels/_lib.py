@@ -146,9 +146,10 @@ SIGNATURES: dict[str, tuple] = {
     ),
 }
 
-# What the wrappers use beside the public entry points (declared in csrc/pa_attention.h).
+# What the wrappers use beside the public entry points; mirrors csrc/pa_internal.h.
 INTERNAL: dict[str, tuple] = {
     "paged_internal_capture_id": (ctypes.c_uint64, [_c_void_p]),
+    "paged_internal_prefill_workspace": (_size_t, [_int, _i32, _i32, _i32, _i32, _i32, _i32]),
 }
 
 _lock = threading.Lock()
@@ -183,7 +184,7 @@ def load() -> ctypes.CDLL:
 def entry_addresses() -> dict[str, int]:
     """Entry point -> address in the loaded library."""
     lib = load()
-    return {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES}
+    return {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES | INTERNAL}
 
 
 def check(status: int, what: str) -> None:

@@ -99,7 +99,8 @@ def _workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
     return ws
 
 
-COUNTER_BYTES = {"decode": 256 << 10}  # PA_DECODE_COUNTER_BYTES in include/paged_hip.h
+# PA_DECODE_COUNTER_BYTES and PA_PREFILL_COUNTER_BYTES in include/paged_hip.h.
+COUNTER_BYTES = {"decode": 256 << 10, "prefill": 64 << 10}
 
 
 def _capture_id(stream: int) -> int:
@@ -132,20 +133,6 @@ def _call_workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tenso
 
 # split_blocks value asking pa_decode for its balanced launch (see include/paged_hip.h).
 DECODE_BALANCED = -1
-
-
-PREFILL_COUNTER_BYTES = 64 << 10  # PA_PREFILL_COUNTER_BYTES in include/paged_hip.h
-
-
-def _prefill_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    """A prefill call's workspace: the kept one on the default stream, where calls follow each other;
-    on other streams, and so under capture, the call's own (its arrival counters zeroed), so that calls
-    on several streams and replays of several graphs never share counters or records."""
-    if _stream_ptr(device) == 0:
-        return _workspace(device, nbytes, "prefill")
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    ws[:PREFILL_COUNTER_BYTES].zero_()
-    return ws
 
 
 def default_split_blocks(batch: int, num_heads: int, max_pages: int, device: torch.device,
@@ -345,6 +332,31 @@ def paged_attention_prefill_hip(
                               PREFILL_BALANCED if split_blocks is None else split_blocks, out)
         if done is not None:
             return done
+    return prefill_in_workspace(None, q, k_pool, v_pool, page_table, seq_lens, current_lengths,
+                                split_blocks=split_blocks, out=out)
+
+
+def prefill_workspace_size(batch: int, num_heads: int, query_len: int, head_dim: int, max_pages: int,
+                           split_blocks: int, kv_dtype: torch.dtype) -> int:
+    """Bytes that a prefill call over KV of one dtype needs (pa_prefill_workspace_size: of either)."""
+    return _lib.load().paged_internal_prefill_workspace(_lib.dtype_code(kv_dtype), batch, num_heads, query_len, head_dim,
+                                                        max_pages, split_blocks)
+
+
+def prefill_in_workspace(
+    ws: torch.Tensor | None,
+    q: torch.Tensor,
+    k_pool: torch.Tensor,
+    v_pool: torch.Tensor,
+    page_table: torch.Tensor,
+    seq_lens: torch.Tensor,
+    current_lengths: torch.Tensor,
+    *,
+    split_blocks: int | None = None,
+    out: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """paged_attention_prefill_hip on a workspace of the caller's (uint8, as long as
+    prefill_workspace_size says, its counters zero and no other call's meanwhile); None: the stream's."""
     _require_gpu("paged_attention_prefill_hip", q, k_pool, v_pool, page_table, seq_lens, current_lengths)
     _check_pool("paged_attention_prefill_hip", k_pool, v_pool)
     B, H, T, Hd = q.shape
@@ -365,9 +377,12 @@ def paged_attention_prefill_hip(
     if split_blocks is None:
         split_blocks = default_prefill_split_blocks(B, H, T, max_pages, q.device, k_pool.dtype)
     lib = _lib.load()
-    ws_bytes = lib.pa_prefill_workspace_size(B, H, T, Hd, max_pages, split_blocks) if bs == 16 else 0
-    ws = _prefill_workspace(q.device, ws_bytes) if ws_bytes else None
-    ws_ptr = ws.data_ptr() if ws is not None else None
+    ws_bytes = prefill_workspace_size(B, H, T, Hd, max_pages, split_blocks, k_pool.dtype) if bs == 16 else 0
+    if ws_bytes and ws is None:
+        ws = _call_workspace(q.device, ws_bytes, "prefill")
+    elif ws_bytes and ws.numel() < ws_bytes:
+        raise ValueError(f"the workspace has {ws.numel()} bytes, the call needs {ws_bytes}")
+    ws_ptr = ws.data_ptr() if ws_bytes else None
     status = lib.pa_prefill(
         q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
         out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), _lib.dtype_code(q.dtype),

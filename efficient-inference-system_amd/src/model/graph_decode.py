@@ -63,7 +63,7 @@ from src.cache.paged_kv import BatchedPagedKVCache, KVStorage
 from src.kernels import _lib, hip_linear
 from src.kernels.hip_paged_attention import (
     _stream_ptr, argmax_rows_hip, decode_in_workspace, default_prefill_split_blocks, default_split_blocks,
-    kv_append_hip, pack_metadata_mirror_hip, paged_attention_prefill_hip)
+    kv_append_hip, pack_metadata_mirror_hip, prefill_in_workspace, prefill_workspace_size)
 from src.kernels.staging import MappedHostWords
 
 try:  # native host bookkeeping (csrc/host/paged_host.cpp): same results as the Python below
@@ -330,17 +330,16 @@ class _Captured:
             self.keys = None
             self.tokens = torch.zeros((B,), dtype=torch.int64, device=device)
         self.last_sel: list[int] = [0] * B
-        lib = _lib.load()
         if Tb == 1:
             self.split_blocks = default_split_blocks(B, H, pages, device)
-            ws_bytes = lib.pa_decode_workspace_size(B, H, Hd, pages, self.split_blocks)
+            ws_bytes = _lib.load().pa_decode_workspace_size(B, H, Hd, pages, self.split_blocks)
         else:
             self.split_blocks = default_prefill_split_blocks(B, H, Tb, pages, device, pools[0].dtype)
-            ws_bytes = lib.pa_prefill_workspace_size(B, H, Tb, Hd, pages, self.split_blocks)
-        # The decode calls' workspace (one after another, layer by layer): this graph's own, so that
+            ws_bytes = prefill_workspace_size(B, H, Tb, Hd, pages, self.split_blocks, pools[0].dtype)
+        # The attention calls' workspace (one after another, layer by layer): this graph's own, so that
         # replays of other graphs and eager calls, on whichever streams, never share it, and zeroed
         # once, outside the capture, since every call leaves its counters zero.
-        self.ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes and Tb == 1 else None
+        self.ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
         self.fused = B * Tb <= FUSED_STEP_ROWS and fused_decode_enabled() and hip_linear.model_supported(model)
         # Steps of at most 16 rows of an fp32 model (every decode step at batch <= 16): per layer
         # four launches, the MLP in one (fc1 column tiles adding their fc2 shares with atomic adds).
@@ -435,8 +434,7 @@ class GraphedStep:
             if Tb == 1:
                 o = decode_in_workspace(cap.ws, q, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
             else:
-                o = paged_attention_prefill_hip(q, k_pool, v_pool, pt, seq32, cap.cur,
-                                                split_blocks=cap.split_blocks)
+                o = prefill_in_workspace(cap.ws, q, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
             x = x + a.out_proj(a.merge_heads(o))
             x = x + blk.mlp(blk.ln2(x))
         return x
@@ -460,7 +458,7 @@ class GraphedStep:
             if Tb == 1:
                 o = decode_in_workspace(cap.ws, q4, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
             else:
-                o = paged_attention_prefill_hip(q4, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
+                o = prefill_in_workspace(cap.ws, q4, k_pool, v_pool, pt, seq32, cap.cur, split_blocks=cap.split_blocks)
             o2 = o.transpose(1, 2).reshape(rows, a.d_model)
             if cap.folded:
                 hip_linear.linear_rows_hip(o2, a.out_proj, residual=x, out=x1_buf, copy_to=x)

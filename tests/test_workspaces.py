@@ -45,12 +45,12 @@ def test_larger_calls_and_the_bound(streams):
     assert (0, 100, "decode") not in hpa._stream_workspaces and streams(7) is b
 
 
-def test_counters_start_at_zero(streams):
-    counters = hpa.COUNTER_BYTES["decode"]
+@pytest.mark.parametrize("kind", ["decode", "prefill"])
+def test_counters_start_at_zero(streams, kind):
     junk = torch.full((1 << 20,), 7, dtype=torch.uint8)  # (whatever memory the allocator hands out next)
     del junk
     for stream in (0, 7):
-        assert int(torch.count_nonzero(streams(stream)[:counters])) == 0
+        assert int(torch.count_nonzero(streams(stream, kind=kind)[:hpa.COUNTER_BYTES[kind]])) == 0
 
 
 def _batch(device, seed, lens, H=8, Hd=64):
@@ -127,28 +127,66 @@ def test_captures_are_told_apart(device):
 
 
 @pytest.mark.gpu
-def test_a_captured_step_has_its_own_workspace(device):
+def test_captured_steps_have_their_own_workspaces(device, monkeypatch):
+    """One per graph, zeroed before the capture: no step takes the stream's or clears counters as it runs."""
     import numpy as np
 
     from src.cache.paged_kv import BatchedPagedKVCache
     from src.model.transformer import TinyTransformerLM
 
+    def taken(*args):
+        raise AssertionError("a captured step took a stream's workspace")
+
     torch.manual_seed(0)
-    model = TinyTransformerLM(64, 256, 4, 2, 512, 1024).to(device).eval()
-    prev = hpa._workspaces.pop((0, "decode"), None)
-    if prev is not None:
-        hpa._retired_workspaces.append(prev)
+    model = TinyTransformerLM(64, 512, 8, 2, 512, 1024).to(device).eval()
     B = 2
     requests = model.create_request_kv_caches(B)
     caches = [BatchedPagedKVCache([requests[r][layer] for r in range(B)], model.layer_block_pools[layer])
               for layer in range(2)]
     ids = np.arange(B * 40).reshape(B, 40) % 64
-    _, _, caches = model.greedy_step(ids, caches, position_offset=0, current_lengths=[40] * B, return_logits=True)
+    step = lambda n, at: model.greedy_step(ids[:, :n].copy(), caches, position_offset=[at] * B,  # noqa: E731
+                                           current_lengths=[n] * B, return_logits=True)
+    step(40, 0)  # (eager: the pools are allocated)
+    monkeypatch.setattr(hpa, "_call_workspace", taken)
+    monkeypatch.setenv("PAGED_HIP_PREFILL_BALANCE", "force")
+    step(40, 40)
     for t in range(3):
-        model.greedy_step(ids[:, :1].copy(), caches, position_offset=[40 + t] * B, current_lengths=[1] * B,
-                          return_logits=True)
-    caps = [c for c in model._graph_step.captured.values() if c.Tb == 1]
-    assert caps and all(c.split_blocks > 0 and c.ws is not None for c in caps)
-    assert (0, "decode") not in hpa._workspaces  # (nothing took the default stream's)
+        step(1, 80 + t)
     torch.cuda.synchronize()
-    assert all(int(torch.count_nonzero(c.ws[:hpa.COUNTER_BYTES["decode"]])) == 0 for c in caps)
+    caps = list(model._graph_step.captured.values())
+    assert sorted(c.Tb for c in caps) == [1, 64]
+    for c in caps:
+        kind = "decode" if c.Tb == 1 else "prefill"
+        assert int(torch.count_nonzero(c.ws[:hpa.COUNTER_BYTES[kind]])) == 0
+    assert len({c.ws.data_ptr() for c in caps}) == 2
+
+
+@pytest.mark.gpu
+def test_prefill_workspace_by_kv_dtype(device):
+    """Where a call over fp32 KV would be balanced and one over bf16 KV is not, the latter takes none."""
+    from src.kernels import _lib
+
+    lib = _lib.load()
+    found = 0
+    for B, H, T, Hd, pages in ((4, 8, 128, 64, 512), (1, 8, 128, 64, 2048), (8, 32, 128, 128, 400), (4, 8, 64, 64, 64)):
+        sizes = [hpa.prefill_workspace_size(B, H, T, Hd, pages, hpa.PREFILL_BALANCED, dt)
+                 for dt in (torch.float32, torch.bfloat16)]
+        assert lib.pa_prefill_workspace_size(B, H, T, Hd, pages, hpa.PREFILL_BALANCED) == max(sizes)
+        if sizes[0] == 0 or sizes[1] > 0:
+            continue
+        found += 1
+        g = torch.Generator(device=device).manual_seed(T)
+        k, v = (torch.randn(64, H, 16, Hd, generator=g, device=device).bfloat16() for _ in range(2))
+        q = torch.randn(B, H, T, Hd, generator=g, device=device)
+        table = torch.randint(0, 64, (B, pages), generator=g, device=device, dtype=torch.int32)
+        lens = torch.full((B,), 300, dtype=torch.int32, device=device)
+        cur = torch.full((B,), T, dtype=torch.int32, device=device)
+        want = hpa.paged_attention_prefill_hip(q, k, v, table, lens, cur, split_blocks=0)
+        st = torch.cuda.Stream()
+        hpa._stream_workspaces.clear()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            got = hpa.paged_attention_prefill_hip(q, k, v, table, lens, cur)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and not hpa._stream_workspaces
+    assert found
