@@ -40,7 +40,7 @@ PyObject* raw_stream = nullptr;  // torch._C._cuda_getCurrentRawStream
 PyObject* fail = nullptr;        // _lib.check(status, what)
 PyObject* side_workspace = nullptr;  // _call_workspace(device, bytes, kind): off the default stream
 PyObject* splits = nullptr;      // default_split_blocks(batch, heads, max_pages, device, ordered)
-PyObject *kind_decode, *kind_prefill, *str_device;
+PyObject *kind_decode, *kind_prefill, *kind_balanced, *str_device;
 
 using Tensor = at::Tensor;
 
@@ -198,13 +198,10 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       if (PyErr_Occurred()) return nullptr;
     }
     const size_t need = t.bs == 16 ? L.decode_ws(t.B, t.H, t.Hd, t.pages, t.split) : 0;
-    Tensor records;  // the balanced launch: this call's own
-    if (need && t.split < 0) records = at::empty({(int64_t)need}, t.q->options().dtype(at::kByte));
     void* stream;
     if (!stream_of(*t.q, stream)) return nullptr;
     Ref held;
-    void* ws = !need ? nullptr
-                     : (t.split < 0 ? records.data_ptr() : workspace(a[0], *t.q, stream, kind_decode, need, held));
+    void* ws = need ? workspace(a[0], *t.q, stream, t.split < 0 ? kind_balanced : kind_decode, need, held) : nullptr;
     if (need && ws == nullptr) return nullptr;
     const Tensor& o = t.result();
     const void* ord = data(order);
@@ -396,6 +393,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_paged_call", "Native front of the
 PyMODINIT_FUNC PyInit__paged_call(void) {
   kind_decode = PyUnicode_InternFromString("decode");
   kind_prefill = PyUnicode_InternFromString("prefill");
+  kind_balanced = PyUnicode_InternFromString("balanced");
   str_device = PyUnicode_InternFromString("device");
-  return kind_decode && kind_prefill && str_device ? PyModule_Create(&module) : nullptr;
+  return kind_decode && kind_prefill && kind_balanced && str_device ? PyModule_Create(&module) : nullptr;
 }

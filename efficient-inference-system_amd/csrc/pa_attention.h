@@ -28,7 +28,8 @@ struct AttnArgs {
   int32_t* counters;     // same-launch merge: arrival counters (zero between calls); decode per
                          // (request, head), balanced wide prefill per (request, head, tile)
   int32_t die_cus;       // balanced wide prefill: compute units per die
-  int32_t balanced;      // decode: balanced launch of num_splits gangs (records in ws, no counters)
+  int32_t balanced;      // decode: balanced launch of num_splits gangs (records in ws, counters: its
+                         // tickets, one uint64_t per (request, head))
 };
 
 // Wave-wide partner exchange on gfx950 without an LDS round trip: v_permlane16_swap /

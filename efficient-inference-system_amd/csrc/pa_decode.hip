@@ -451,16 +451,22 @@ __global__ __launch_bounds__(kWave) void decode_merge_kernel(const AttnArgs a) {
 // keys counts as one block), are dealt out evenly: gang g takes positions [W g / NG, W (g + 1) / NG)
 // of the list's W, walking the part of every request in its share. A request cut by a share's end
 // leaves one (m, l, acc) record per gang and head, in slot 0 (the share's first request) or 1 (its
-// last), merged in gang order by decode_balanced_merge_kernel; the others are written directly.
+// last); the gang that arrives last merges them, in gang order. Where that would gain nothing, no request
+// is cut and gang g takes requests g, g + NG, ... whole: where the longest gang would then walk at
+// most kTailBlocks more than the mean (about what records, arrival and merge cost, 4 us), if at least
+// half of the gangs have a request or no request is longer than that.
 //   bound: HBM. One workgroup per (request, head) leaves the longest contexts running alone at the
 //   end, and a fixed split size costs every batch records and, where the lengths turn out short, empty
 //   workgroups (a second round of them took 5% of a uniform batch). Here the number of pieces is
-//   that of the gangs and every batch ends at once. MI355X, 16 requests x 32 heads x 128 bf16 over
-//   lengths log-uniform in 512 .. 32768, one workgroup per pair -> balanced: 363 -> 324 us (5.8 ->
-//   6.5 TB/s); 64 x 8 heads x 64 fp32 455 -> 307; 16 equal contexts of 32768 1270 -> 1275 (6.8).
+//   that of the gangs and every batch ends at once. MI355X, in a graph, 16 requests x 32 heads x 128
+//   bf16 over lengths log-uniform in 512 .. 32768, one workgroup per pair -> balanced: 453 -> 326 us
+//   (6.5 TB/s); 64 x 8 heads x 64 fp32 524 -> 317; 16 equal contexts of 32768 1330 -> 1306. A table as
+//   wide over short requests (uncut): 16 x 32 x 128 bf16 at up to 64 and 256 tokens 4.4 -> 6.1 and 8.7 ->
+//   10.1 us, 8 x 32 x 128 (32-block splits before) 5.0 -> 5.0 and 9.0 -> 8.3; with a second launch
+//   for the merge and every request cut it was 13.0, 17.2, 11.1 and 13.5.
 // ---------------------------------------------------------------------------------------------
 constexpr int kBalancedMaxBatch = 512;
-constexpr int kDecodeMergeHd = 128;  // largest head_dim of the fast kernels
+constexpr int kTailBlocks = 32;
 
 // List positions: the blocks request b counts for.
 __device__ __forceinline__ int balanced_blocks(const AttnArgs& a, int b) {
@@ -475,6 +481,24 @@ __device__ __forceinline__ int share_of(int W, int NG, int pos) {
   return (int)((((int64_t)pos + 1) * NG - 1) / W);
 }
 
+// Arrivals at a cut request, counted in a ticket word that needs no initial state: a word without the
+// mark (as its upper half a signalling NaN, which no arithmetic leaves in a record) stands for zero
+// arrivals, the first to come marks it, and the last of `pieces` leaves a marked zero. `seen`: the word
+// at any earlier time of the launch (marked words stay marked). True for the last to arrive.
+constexpr uint64_t kTicketMark = 0x7FA5C3E15A7Cull;
+__device__ __forceinline__ bool arrive_last(uint64_t* ticket, int pieces, uint64_t seen) {
+  // (an exchange fails only because another arrival has marked the word)
+  while ((seen >> 16) != kTicketMark) {
+    if (__hip_atomic_compare_exchange_strong(ticket, &seen, (kTicketMark << 16) | 1, __ATOMIC_RELAXED,
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      return false;  // (a cut request has at least two pieces)
+  }
+  seen = __hip_atomic_fetch_add(ticket, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((int)(seen & 0xffff) + 1 < pieces) return false;
+  __hip_atomic_store(ticket, kTicketMark << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
 template <typename KV, typename IO, int HD, int NW>
 __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(sizeof(KV) == 4 && HD == 128 ? 2 : 4)))
 void decode_balanced_kernel(const AttnArgs a) {
@@ -486,22 +510,31 @@ void decode_balanced_kernel(const AttnArgs a) {
   __shared__ float sm_m[NW];
   __shared__ float sm_l[NW];
   __shared__ int sS[kBalancedMaxBatch + 1];  // list position of each request's first block
-  __shared__ int sWave[NW];
+  __shared__ int sWave[NW], sMost[NW];
+  __shared__ int sm_last[2];
 
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int gang = blockIdx.x / a.H;
   const int h = blockIdx.x - gang * a.H;
+  int most;  // blocks of the longest request
   {  // prefix sums: shuffles inside a wavefront, then the wavefronts' totals
     int x = (int)threadIdx.x < a.B ? balanced_blocks(a, threadIdx.x) : 0;
+    most = x;
 #pragma unroll
     for (int off = 1; off < kWave; off <<= 1) {
       const int y = __shfl_up(x, off);
       if (lane >= off) x += y;
+      const int z = __shfl_xor(most, off);
+      most = most > z ? most : z;
     }
-    if (lane == kWave - 1) sWave[w] = x;
+    if (lane == kWave - 1) {
+      sWave[w] = x;
+      sMost[w] = most;
+    }
     __syncthreads();
     for (int ww = 0; ww < w; ++ww) x += sWave[ww];
+    for (int ww = 0; ww < NW; ++ww) most = most > sMost[ww] ? most : sMost[ww];
     if ((int)threadIdx.x < a.B) sS[threadIdx.x + 1] = x;
     if (threadIdx.x == 0) sS[0] = 0;
     __syncthreads();
@@ -509,17 +542,61 @@ void decode_balanced_kernel(const AttnArgs a) {
   const int W = __builtin_amdgcn_readfirstlane(sS[a.B]);
   const int NG = a.num_splits < W ? a.num_splits : W;
   if (gang >= NG) return;  // uniform over the workgroup
-  const int lo = share_start(W, NG, gang), hi = share_start(W, NG, gang + 1);
+  most = __builtin_amdgcn_readfirstlane(most);
+  const int busy = a.B < NG ? a.B : NG;
+  const bool uncut = (a.B + NG - 1) / NG * most - W / busy <= kTailBlocks && (2 * busy >= NG || most <= kTailBlocks);
+  int lo = share_start(W, NG, gang), hi = share_start(W, NG, gang + 1);
   int b = 0;
-  for (int ub = a.B - 1; b < ub;) {
-    const int mid = (b + ub + 1) / 2;
-    if (__builtin_amdgcn_readfirstlane(sS[mid]) <= lo) b = mid;
-    else ub = mid - 1;
+  if (uncut) {
+    b = gang;
+  } else {
+    for (int ub = a.B - 1; b < ub;) {
+      const int mid = (b + ub + 1) / 2;
+      if (__builtin_amdgcn_readfirstlane(sS[mid]) <= lo) b = mid;
+      else ub = mid - 1;
+    }
   }
+  // The wavefronts' states as one: put(d, M, l, acc[d]).
+  auto combined = [&](auto&& put) {
+    float M = kNegBig;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, sm_m[ww]);
+    for (int d = threadIdx.x; d < HD; d += NW * kWave) {
+      float lsum = 0.f, A = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) {
+        const float f = fast_exp2(sm_m[ww] - M);
+        lsum = fmaf(sm_l[ww], f, lsum);
+        A = fmaf(sm_acc[ww][d], f, A);
+      }
+      put(d, M, lsum, A);
+    }
+  };
+  auto write = [&](int req) {
+    combined([&](int d, float, float lsum, float A) {
+      IO* op = static_cast<IO*>(a.out) + (int64_t)req * a.o_sb + (int64_t)h * a.o_sh;
+      Elem<IO>::store(op + d, lsum > 0.f ? A / lsum : 0.f);
+    });
+  };
+  // Gang g's record of the request at position `first`: slot 0, or 1 where its share starts earlier.
+  constexpr int R = HD + 2;
+  auto record = [&](int g, int first) {
+    return a.ws + (((int64_t)g * a.H + h) * 2 + (share_start(W, NG, g) >= first ? 0 : 1)) * R;
+  };
+  uint64_t* tickets = reinterpret_cast<uint64_t*>(a.counters);
+  int cuts = 0, cut[2] = {0, 0};  // this share's cut requests: its first, its last or both
+  uint64_t seen = 0;              // thread 0: the ticket of the first of them, thread kWave: of the second
   const int r = lane % LPR;
-  for (; b < a.B; ++b) {
+  for (; b < a.B; b += uncut ? NG : 1) {
     const int first = __builtin_amdgcn_readfirstlane(sS[b]), end = __builtin_amdgcn_readfirstlane(sS[b + 1]);
+    if (uncut) {
+      lo = first;
+      hi = end;
+    }
     if (first >= hi) break;
+    const bool whole = lo <= first && hi >= end;
+    if (!whole && (int)threadIdx.x == cuts * kWave)
+      seen = __hip_atomic_load(tickets + (int64_t)b * a.H + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int n = valid_keys(a.seq_lens[b], a.cur_lens[b], 0);
     const int nb = n > 0 ? end - first : 0;  // (a.max_pages == 0: one position, no block)
     const int jb = lo > first ? lo - first : 0;
@@ -538,80 +615,80 @@ void decode_balanced_kernel(const AttnArgs a) {
     for (int e = 0; e < EPL; ++e) qv[e] = Elem<IO>::load(qp + e) * a.scale_log2;
     walk_blocks<KV, HD, NW>(a, pt, h, jb, je, n, ids0, w, lane, qv, sm_acc, sm_m, sm_l);
     __syncthreads();
-    const bool whole = lo <= first && hi >= end;
-    float M = kNegBig;
-#pragma unroll
-    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, sm_m[ww]);
-    for (int d = threadIdx.x; d < HD; d += NW * kWave) {
-      float lsum = 0.f, A = 0.f;
-#pragma unroll
-      for (int ww = 0; ww < NW; ++ww) {
-        const float f = fast_exp2(sm_m[ww] - M);
-        lsum = fmaf(sm_l[ww], f, lsum);
-        A = fmaf(sm_acc[ww][d], f, A);
-      }
-      if (whole) {
-        IO* op = static_cast<IO*>(a.out) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
-        Elem<IO>::store(op + d, lsum > 0.f ? A / lsum : 0.f);
-      } else {
-        float* rec = a.ws + (((int64_t)gang * a.H + h) * 2 + (lo >= first ? 0 : 1)) * (HD + 2);
+    if (whole) {
+      write(b);
+    } else {
+      float* mine = record(gang, first);
+      combined([&](int d, float M, float lsum, float A) {
         if (d == 0) {
-          rec[0] = M;
-          rec[1] = lsum;
+          __hip_atomic_store(mine, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(mine + 1, lsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        rec[2 + d] = A;
-      }
+        __hip_atomic_store(mine + 2 + d, A, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      });
+      cut[cuts] = b;
+      ++cuts;
     }
     __syncthreads();  // the next request's states go to the same LDS
   }
-}
-
-// Merge of the requests cut by the balanced launch: one wavefront per (request, head).
-template <typename IO>
-__global__ __launch_bounds__(kWave) void decode_balanced_merge_kernel(const AttnArgs a) {
-  const int lane = threadIdx.x;
-  const int b = blockIdx.x / a.H, h = blockIdx.x - b * a.H;
-  int before = 0, total = 0, mine = 0;
-  for (int r = lane; r < a.B; r += kWave) {
-    const int p = balanced_blocks(a, r);
-    total += p;
-    before += r < b ? p : 0;
-    mine += r == b ? p : 0;
-  }
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    total += __shfl_xor(total, off);
-    before += __shfl_xor(before, off);
-    mine += __shfl_xor(mine, off);
-  }
-  const int W = __builtin_amdgcn_readfirstlane(total), first = __builtin_amdgcn_readfirstlane(before);
-  const int NG = a.num_splits < W ? a.num_splits : W;
-  const int g0 = share_of(W, NG, first);
-  const int g1 = share_of(W, NG, first + __builtin_amdgcn_readfirstlane(mine) - 1);
-  if (g0 == g1) return;  // written whole
-  const int HD = a.head_dim;
-  const int64_t R = HD + 2;
-  // Gang g's record: slot 0, or 1 where its share starts in an earlier request (only g0's can).
-  auto rec = [&](int g) {
-    return a.ws + (((int64_t)g * a.H + h) * 2 + (share_start(W, NG, g) >= first ? 0 : 1)) * R;
+  if (cuts == 0) return;
+  // The gang arrives at its cut requests, once every wavefront's record stores have completed at
+  // device scope, and merges those that it is the last to arrive at.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  auto pieces = [&](int req, int& g0) {
+    g0 = share_of(W, NG, sS[req]);
+    return share_of(W, NG, sS[req + 1] - 1) - g0 + 1;
   };
-  float M = kNegBig;
-  for (int g = g0 + lane; g <= g1; g += kWave) M = fmaxf(M, rec(g)[0]);
-  M = wave_max(M);
-  float lsum = 0.f, A[kDecodeMergeHd / kWave] = {};
-  for (int g = g0; g <= g1; ++g) {
-    const float* x = rec(g);
-    const float f = fast_exp2(x[0] - M);
-    lsum = fmaf(x[1], f, lsum);
-#pragma unroll
-    for (int t = 0; t < kDecodeMergeHd / kWave; ++t)
-      if (lane + t * kWave < HD) A[t] = fmaf(x[2 + lane + t * kWave], f, A[t]);
+  if (lane == 0 && w < cuts) {
+    const int req = w == 0 ? cut[0] : cut[1];
+    int g0;
+    const int np = pieces(req, g0);
+    sm_last[w] = arrive_last(tickets + (int64_t)req * a.H + h, np, seen);
   }
-  IO* op = static_cast<IO*>(a.out) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
-  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+  __syncthreads();
+  for (int c = 0; c < cuts; ++c) {
+    if (!__builtin_amdgcn_readfirstlane(sm_last[c])) continue;
+    const int req = c == 0 ? cut[0] : cut[1];
+    int g0;
+    const int np = __builtin_amdgcn_readfirstlane(pieces(req, g0));
+    g0 = __builtin_amdgcn_readfirstlane(g0);
+    const int first = __builtin_amdgcn_readfirstlane(sS[req]);
+    // Wavefront w folds records w, w + NW, ... four at a time, their words all in flight.
+    static_assert(HD % kWave == 0, "whole lanes");
+    constexpr int DL = HD / kWave;
+    float m = kNegBig, l = 0.f, acc[DL] = {};
+    for (int p = w; p < np; p += 4 * NW) {
+      float rm[4], rl[4], ra[4][DL];
 #pragma unroll
-  for (int t = 0; t < kDecodeMergeHd / kWave; ++t)
-    if (lane + t * kWave < HD) Elem<IO>::store(op + lane + t * kWave, A[t] * inv);
+      for (int t = 0; t < 4; ++t) {
+        const float* x = record(g0 + (p + t * NW < np ? p + t * NW : np - 1), first);
+        rm[t] = rec_load<true>(x);
+        rl[t] = rec_load<true>(x + 1);
+#pragma unroll
+        for (int e = 0; e < DL; ++e) ra[t][e] = rec_load<true>(x + 2 + lane + e * kWave);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (p + t * NW >= np) break;
+        const float mn = fmaxf(m, rm[t]);
+        const float fa = fast_exp2(m - mn), fr = fast_exp2(rm[t] - mn);
+        l = l * fa + rl[t] * fr;
+#pragma unroll
+        for (int e = 0; e < DL; ++e) acc[e] = acc[e] * fa + ra[t][e] * fr;
+        m = mn;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < DL; ++e) sm_acc[w][lane + e * kWave] = acc[e];
+    if (lane == 0) {
+      sm_m[w] = m;
+      sm_l[w] = l;
+    }
+    __syncthreads();
+    write(req);
+    __syncthreads();
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -775,16 +852,24 @@ using namespace pa;
 // Split workspace layout: arrival counters (one int32 per (request, head), at most
 // kDecodeCounterBytes / 4 pairs) at the start, zero between calls, then the split records. The
 // counters region has one fixed size whatever the call's shape, so calls of any shapes can share
-// a workspace and always find their counters at zero. The balanced launch's records lie behind that
-// region too, which it neither reads nor writes.
+// a workspace and always find their counters at zero. The balanced launch's tickets (one 8-byte word
+// per (request, head)) and records lie behind that region, which it neither reads nor writes.
 constexpr size_t kDecodeCounterBytes = PA_DECODE_COUNTER_BYTES;
 // Splits per (request, head) up to which the last split to finish merges the records in the same
 // launch; more splits are merged by a second launch (its merge reads them faster than one
 // workgroup's device-scope loads).
 constexpr int kSameLaunchMaxSplits = 8;
 
-static size_t balanced_workspace(int gangs, int32_t num_heads, int32_t head_dim) {
-  return gangs > 0 ? kDecodeCounterBytes + (size_t)gangs * num_heads * 2 * (head_dim + 2) * sizeof(float) : 0;
+// Room for the tickets: the same for all calls of up to 32768 pairs, so that calls of other shapes on one
+// workspace find them marked (not overwritten by records, which costs an exchange each).
+static size_t ticket_bytes(int32_t batch, int32_t num_heads) {
+  const size_t need = (size_t)batch * num_heads * sizeof(uint64_t), fixed = (size_t)256 << 10;
+  return need > fixed ? need : fixed;
+}
+static size_t balanced_workspace(int gangs, int32_t batch, int32_t num_heads, int32_t head_dim) {
+  return gangs > 0 ? kDecodeCounterBytes + ticket_bytes(batch, num_heads) +
+                         (size_t)gangs * num_heads * 2 * (head_dim + 2) * sizeof(float)
+                   : 0;
 }
 
 extern "C" size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int32_t head_dim,
@@ -797,7 +882,7 @@ extern "C" size_t pa_decode_workspace_size(int32_t batch, int32_t num_heads, int
         const int x = balanced_gangs(batch, num_heads, head_dim, max_pages, io, kv);
         g = x > g ? x : g;
       }
-    return balanced_workspace(g, num_heads, head_dim);
+    return balanced_workspace(g, batch, num_heads, head_dim);
   }
   const int s = num_splits_for(max_pages, split_blocks);
   if (s <= 1 || batch <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
@@ -846,12 +931,15 @@ static int decode_entry(const void* q, int64_t q_stride_b, int64_t q_stride_h,
   int gangs = 0;
   if (split_blocks < 0 && workspace != nullptr && !ws_limit_is_scratch) {
     gangs = balanced_gangs(batch, num_heads, head_dim, max_pages, io_dtype, kv_dtype);
-    if (workspace_bytes < balanced_workspace(gangs, num_heads, head_dim)) gangs = 0;  // unsplit
+    if (workspace_bytes < balanced_workspace(gangs, batch, num_heads, head_dim) ||
+        (reinterpret_cast<uintptr_t>(workspace) & 7) != 0)  // (the tickets are 8-byte words)
+      gangs = 0;  // unsplit
   }
   const int nsplit = num_splits_for(max_pages, split_blocks);
   if (gangs > 0) {
     a.num_splits = gangs;
-    a.ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + kDecodeCounterBytes);
+    a.counters = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + kDecodeCounterBytes);
+    a.ws = reinterpret_cast<float*>(reinterpret_cast<char*>(a.counters) + ticket_bytes(batch, num_heads));
     a.balanced = 1;
   } else if (nsplit > 1) {
     const size_t need = pa_decode_workspace_size(batch, num_heads, head_dim, max_pages, split_blocks);
@@ -875,14 +963,7 @@ static int decode_entry(const void* q, int64_t q_stride_b, int64_t q_stride_h,
                                            : dispatch_decode_fast_io<uint16_t>(a, kv_dtype, stream);
   if (!ok) PA_FAIL(PA_ERR_UNSUPPORTED, "no decode kernel for head_dim %d", head_dim);
   PA_CHECK_LAUNCH("decode kernel");
-  if (gangs > 0) {
-    const dim3 grid((unsigned)((int64_t)batch * num_heads)), block(kWave);
-    if (io_dtype == PA_DTYPE_F32)
-      decode_balanced_merge_kernel<float><<<grid, block, 0, stream>>>(a);
-    else
-      decode_balanced_merge_kernel<uint16_t><<<grid, block, 0, stream>>>(a);
-    PA_CHECK_LAUNCH("balanced decode merge kernel");
-  } else if (nsplit > 1 && a.counters == nullptr) {
+  if (gangs == 0 && nsplit > 1 && a.counters == nullptr) {
     const dim3 grid((unsigned)((int64_t)batch * num_heads)), block(kWave);
     if (io_dtype == PA_DTYPE_F32)
       decode_merge_kernel<float><<<grid, block, 0, stream>>>(a);

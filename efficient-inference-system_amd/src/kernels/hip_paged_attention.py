@@ -31,7 +31,7 @@ _retired_workspaces: list[torch.Tensor] = []
 # Workspaces off the default stream: (device, stream, kind) -> (capture, tensor), the latest used last.
 _stream_workspaces: dict[tuple[int, int, str], tuple[int, torch.Tensor]] = {}
 _stream_workspaces_lock = threading.Lock()
-MAX_STREAM_WORKSPACES = 8
+MAX_STREAM_WORKSPACES = 16
 _cu_counts: dict[int, int] = {}
 
 
@@ -84,10 +84,10 @@ def cu_count(device: torch.device) -> int:
 
 
 def _workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
-    """The default stream's split-K workspace for `kind` ("decode" or "prefill"), at least `nbytes` long.
-    Both kinds start with arrival counters of the in-launch merges, which must be zero before first
-    use and stay zero between calls: workspaces are zero-filled when allocated, and the two kinds
-    are kept apart (their layouts differ). A workspace replaced by a larger one stays allocated
+    """The default stream's split-K workspace for `kind` ("decode", "prefill", or "balanced" decode), at
+    least `nbytes` long. The first two start with arrival counters of the in-launch merges, which must
+    be zero before first use and stay zero between calls: workspaces are zero-filled when allocated,
+    and the kinds are kept apart (their layouts differ). A workspace replaced by a larger one stays allocated
     for the life of the process: a HIP graph a caller captured may hold its address."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
     ws = _workspaces.get((idx, kind))
@@ -100,7 +100,8 @@ def _workspace(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
 
 
 # PA_DECODE_COUNTER_BYTES and PA_PREFILL_COUNTER_BYTES in include/paged_hip.h.
-COUNTER_BYTES = {"decode": 256 << 10, "prefill": 64 << 10}
+# (A balanced decode needs no initial state, but finds its tickets faster where it left them.)
+COUNTER_BYTES = {"decode": 256 << 10, "prefill": 64 << 10, "balanced": 0}
 
 
 def _capture_id(stream: int) -> int:
@@ -147,13 +148,13 @@ def default_split_blocks(batch: int, num_heads: int, max_pages: int, device: tor
     32-block splits against 74 / 75 / 83 us unsplit.
 
     DECODE_BALANCED above 128 pairs where contexts may pass 8192 tokens: it ends every workgroup at
-    once whatever the lengths. Against the rules above, heads x head_dim, lengths log-uniform / equal:
-    16 x 32 x 128 bf16 to 32k 363 -> 324 us / 1270 -> 1275; 64 x 32 x 128, bf16 KV, to 32k 1360 -> 1226;
-    8 x 32 x 128 to 32k 188 -> 155, to 8k 57 -> 53 / 168 -> 170; 64 x 8 x 64 fp32 to 32k 455 -> 307;
-    32 x 8 x 64 fp32 to 32k 313 -> 160; 20 x 8 x 64, bf16 KV, to 32k 83 -> 57 / at 8k 57 -> 58. At 4096
-    tokens its second launch (4.5 us) takes what it gains (equal lengths 163 -> 168, others within
-    1%), and with eight pairs per compute unit in the caller's order (longest first) the grid's end
-    is already filled with short contexts (1214 against 1226)."""
+    once whatever the lengths. Against the rules above, heads x head_dim, lengths log-uniform from 512 /
+    equal, in a graph: 16 x 32 x 128 bf16 to 32k 453 -> 326 us / 1330 -> 1306; 64 x 32 x 128, bf16 KV, to 32k
+    1339 -> 1271; 8 x 32 x 128 to 32k 305 -> 173, at 8k 171 -> 169; 64 x 8 x 64 fp32 to 32k 524 -> 317;
+    32 x 8 x 64 fp32 to 32k 306 -> 158; 20 x 8 x 64, bf16 KV, to 32k 88 -> 58 / at 8k 58 -> 60. Tables this wide
+    over contexts of at most 256 tokens: 16 x 32 x 128 8.7 -> 10.1, 8 x 32 x 128 9.0 -> 8.3, 32 x 8 x 64 7.5 ->
+    7.0, 64 x 8 x 64 8.1 -> 9.0. With eight pairs per compute unit in the caller's order (longest first)
+    the grid's end is already filled with short contexts (1214 against 1226)."""
     units = batch * num_heads
     target = 2 * cu_count(device)
     if units > 128 and max_pages >= 512 and batch <= 512 and not (ordered and units >= 4 * target):
@@ -292,9 +293,8 @@ def decode_in_workspace(
         split_blocks = default_split_blocks(B, H, max_pages, q.device, order is not None)
     lib = _lib.load()
     ws_bytes = lib.pa_decode_workspace_size(B, H, Hd, max_pages, split_blocks) if bs == 16 else 0
-    if ws_bytes and ws is None:  # (the balanced launch: records only, this call's own)
-        ws = _call_workspace(q.device, ws_bytes, "decode") if split_blocks > 0 else \
-            torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+    if ws_bytes and ws is None:
+        ws = _call_workspace(q.device, ws_bytes, "decode" if split_blocks > 0 else "balanced")
     elif ws_bytes and ws.numel() < ws_bytes:
         raise ValueError(f"the workspace has {ws.numel()} bytes, the call needs {ws_bytes}")
     ws_ptr = ws.data_ptr() if ws_bytes else None

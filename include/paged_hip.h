@@ -74,12 +74,14 @@ const char* pa_last_error_message(void);
  * allocation serves all later calls of any shape; other calls (pa_prefill) must not write into
  * that region. split_blocks == 0 means one workgroup per (request, head) and no workspace.
  * split_blocks < 0 asks for the balanced launch (at most 512 requests; other calls run unsplit): as many
- * workgroups as the GPU holds share the requests' KV blocks evenly whatever their lengths, and a
- * second kernel merges the requests that a share's end cuts. Its workspace of
- * pa_decode_workspace_size() bytes holds records behind PA_DECODE_COUNTER_BYTES that it leaves
- * alone: it needs no initial state, may be freed or reused, in stream order, after the call, and, if
- * zeroed once, serves split calls (split_blocks > 0) as well, in any order. Without a workspace, or
- * with a smaller one, such a call runs unsplit. The balanced launch does not use order.
+ * workgroups as the GPU holds share the requests' KV blocks evenly whatever their lengths, and the
+ * one that finishes a request cut by a share's end last merges it, in the same launch. Its workspace
+ * of pa_decode_workspace_size() bytes holds arrival tickets and records behind
+ * PA_DECODE_COUNTER_BYTES that it leaves alone: it needs no initial state (memory that the last such
+ * call used is a little faster), may be freed or reused, in stream order, after the call, and, if
+ * zeroed once, serves split calls (split_blocks > 0) as well, in any order. Without a workspace, with
+ * a smaller one or one that is not 8-byte aligned, such a call runs unsplit. The balanced launch does
+ * not use order.
  *
  * order: optional int32 [B] permutation giving the processing order of requests (e.g. longest
  * first, for load balance); NULL means 0..B-1. Results do not depend on it.
@@ -93,8 +95,9 @@ int pa_decode(const void* q, int64_t q_stride_b, int64_t q_stride_h,
               float scale, int32_t split_blocks,
               void* workspace, size_t workspace_bytes, void* stream);
 
-/* Bytes of workspace pa_decode needs for these sizes (split_blocks < 0: PA_DECODE_COUNTER_BYTES and two
- * records per workgroup of the balanced launch on the current device, 0 where it does not apply;
+/* Bytes of workspace pa_decode needs for these sizes (split_blocks < 0: PA_DECODE_COUNTER_BYTES, the
+ * tickets and two records per workgroup of the balanced launch on the current device, 0 where it does
+ * not apply;
  * otherwise 0 when split_blocks == 0 or no request can need more than one split, else
  * PA_DECODE_COUNTER_BYTES + 4 * batch * num_heads * splits * (head_dim + 2)). No reference counterpart: the Triton decode path has no split-K.
  * Calls that share a workspace must not run concurrently (e.g. on different streams). */

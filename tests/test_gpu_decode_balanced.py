@@ -29,7 +29,7 @@ def _batch(device, lens, H, Hd, io, kv, seed=0, extra_pages=3):
     return (q, k, v, table, seq, torch.ones_like(seq)), lists
 
 
-LENS = [[1], [4000], [0, 0, 0], [0, 5, 0, 300, 16, 17], [16] * 70, [2000, 1, 1, 1, 900], list(range(1, 513)),
+LENS = [[512] * 40, [513] + [512] * 39, [300, 5] * 100, [1], [4000], [0, 0, 0], [0, 5, 0, 300, 16, 17], [16] * 70, [2000, 1, 1, 1, 900], list(range(1, 513)),
         [333] * 31 + [7000]]
 
 
@@ -148,3 +148,54 @@ def test_a_workspace_too_small_for_the_records_runs_unsplit(device):
         out = torch.full_like(dev[0], 9.0)
         assert _entry(lib, dev, out, DECODE_BALANCED, ws, nbytes) == 0, lib.pa_last_error_message()
         assert torch.equal(out, want) and int(torch.count_nonzero(ws)) == 0
+
+
+@pytest.mark.parametrize("fill", ["random", "ones", "earlier call"])
+def test_any_state_of_the_workspace(device, fill):
+    """The tickets and records need no initial state: noise, all ones, or what a call of another shape left."""
+    lib = _lib.load()
+    cases = [[t.to(device) for t in _batch(device, lens, H, Hd, torch.float32, kv, 5)[0]]
+             for lens, H, Hd, kv in (([3000, 1, 700, 2500], 8, 64, torch.float32),
+                                     ([900] * 30 + [6000], 32, 128, torch.bfloat16), ([1500, 700], 3, 64, torch.float32))]
+    size = max(lib.pa_decode_workspace_size(c[0].shape[0], c[0].shape[1], c[0].shape[3], c[3].shape[1], DECODE_BALANCED)
+               for c in cases)
+    ws = torch.zeros(size, dtype=torch.uint8, device=device)
+    want = [paged_attention_decode_hip(*c, split_blocks=0) for c in cases]
+    first = [None] * 3
+    for rep in range(3):
+        for i, c in enumerate(cases):
+            if fill == "random":
+                ws.random_(0, 256)
+            elif fill == "ones":
+                ws.fill_(255)
+            out = torch.full_like(c[0], 9.0)
+            assert _entry(lib, c, out, DECODE_BALANCED, ws, size) == 0
+            assert float((out - want[i]).abs().max()) <= 4e-6, (rep, i)  # (as test_same_as_unsplit)
+            assert rep == 0 or torch.equal(out, first[i])  # whichever gang arrives last
+            first[i] = out
+
+
+@pytest.mark.parametrize("lens", [[40] * 16, [9000, 30, 700, 2500] * 4], ids=["short", "long"])
+def test_one_launch(device, lens):
+    """A balanced call is one kernel, whatever it has to merge: a server that hands one wide table for short
+    contexts pays for no second one."""
+    import ctypes
+    from pathlib import Path
+
+    hip = ctypes.CDLL(str(Path(torch.__file__).parent / "lib" / "libamdhip64.so"))
+    dev = [t.to(device) for t in _batch(device, lens, 32, 128, torch.bfloat16, torch.bfloat16, extra_pages=600)[0]]
+    out = torch.empty_like(dev[0])
+    want = paged_attention_decode_hip(*dev, out=torch.empty_like(out)).clone()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        assert default_split_blocks(len(lens), 32, dev[3].shape[1], device) == DECODE_BALANCED
+        paged_attention_decode_hip(*dev, out=out)
+    nodes = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    assert nodes.value == 1
+    graph.instantiate()
+    for _ in range(2):
+        out.fill_(9.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
