@@ -658,9 +658,13 @@ void prefill_wide_kernel(const AttnArgs a) {
           if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           // Gang gg's record is in its slot 0, except gang g0's when its share starts before the
           // tile (the tile is then its share's last pair: slot 1).
-          if (gang != g0) {
+          if (gang != g0) {  // (from nothing: its own piece comes back as a record; 0 * inf would be NaN)
             m = kNegBig;
             l = 0.f;
+#pragma unroll
+            for (int d = 0; d < DU; ++d)
+#pragma unroll
+              for (int e = 0; e < 16; ++e) oacc[d][e] = 0.f;
           }
           for (int gg = gang == g0 ? g0 + 1 : g0; gg < g0 + np; ++gg) {
             const int slot = __builtin_amdgcn_readfirstlane(sLo[gg]) >= tile_start ? 0 : 1;
@@ -1200,9 +1204,13 @@ void prefill_wide_f32_kernel(const AttnArgs a) {
       store = last;
       if (last) {
         if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (gang != g0) {
+        if (gang != g0) {  // (from nothing: its own piece comes back as a record; 0 * inf would be NaN)
           m = kNegBig;
           l = 0.f;
+#pragma unroll
+          for (int d = 0; d < DU; ++d)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) oacc[d][e] = 0.f;
         }
         for (int gg = gang == g0 ? g0 + 1 : g0; gg < g0 + np; ++gg) {
           const int slot = __builtin_amdgcn_readfirstlane(sLo[gg]) >= tile_start ? 0 : 1;
