@@ -74,7 +74,15 @@ def test_qkv_scatter(device, monkeypatch, dtype, pool):
         assert float((a.float() - b.float()).norm() / b.float().norm()) < (4e-3 if low else 1e-6)
 
 
-@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3e38, -2.0**61])
+def _same(got, want, rel):
+    """Numbers to a relative error, infinities and NaNs by themselves."""
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
+    ok = want.isfinite()
+    assert float((got - want)[ok].norm()) <= rel * float(want[ok].norm())
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3e38, -2.0**61])
 @torch.no_grad()
 def test_values_without_a_finite_split(device, monkeypatch, value):
     """In the weights (one output column) and in the rows (one row): only what they reach differs."""
@@ -85,27 +93,67 @@ def test_values_without_a_finite_split(device, monkeypatch, value):
     lin.weight[7, 11] = value
     got, want = linear_rows_hip(x, lin, ln=ln), _want(x, lin, ln).float()
     keep = torch.arange(N, device=device) != 7
-    assert float((got[:, keep] - want[:, keep]).norm() / want[:, keep].norm()) < 1e-6
-    both = got[:, 7].isfinite() & want[:, 7].isfinite()
-    assert torch.equal(got[:, 7].isfinite(), want[:, 7].isfinite())
-    if bool(both.any()):
-        assert float(((got - want)[:, 7][both] / want[:, 7][both]).abs().max()) < 1e-4
+    _same(got[:, keep], want[:, keep], 1e-6)
+    _same(got[:, 7], want[:, 7], 1e-6)
     lin.weight[7, 11] = 0.1
     x[140, 3] = value
     got, want = linear_rows_hip(x, lin, ln=ln), _want(x, lin, ln).float()
     keep = torch.arange(M, device=device) != 140
-    assert float((got[keep] - want[keep]).norm() / want[keep].norm()) < 1e-6
+    _same(got[keep], want[keep], 1e-6)
+    if abs(value) < 1e19:  # (the row's variance is an fp32 number)
+        _same(got[140], want[140], 1e-6)
+    elif not abs(value) < float("inf"):
+        assert bool(got[140].isnan().all())
 
 
-@pytest.mark.parametrize("rows", [575, 576, 577, 800])
+@pytest.mark.parametrize("where", ["weight", "norm"])
+@pytest.mark.parametrize("value", [3.4028234663852886e38, -3.4028234663852886e38, 3e37])
 @torch.no_grad()
-def test_default_choice_near_its_line(device, monkeypatch, rows):
-    """fc1-shaped layers around four and a half tiled workgroups per compute unit (576 rows on 256)."""
-    monkeypatch.delenv("PAGED_HIP_LINEAR_KERNEL", raising=False)
+def test_values_that_only_fp32_products_hold(device, monkeypatch, where, value):
+    """Finite results from values whose parts are not finite: the products are formed again in fp32, or the
+    outputs would be NaN. The other operand is small enough for every product to be finite."""
+    assert torch.tensor(value * 2.0**24, dtype=torch.float64).bfloat16().isinf()  # (the leading part)
+    monkeypatch.setenv("PAGED_HIP_LINEAR_KERNEL", "block")
+    M, N = 150, 130
+    lin, ln = _layer(N, torch.float32, device, 3)
+    x = torch.randn(M, K, device=device)
+    if where == "weight":
+        ln.weight[11], ln.bias[11] = 1e-3, 0.0
+        lin.weight[7, 11] = value
+    else:
+        ln.weight[11], ln.bias[11] = value / 8, 0.0  # (rows of up to 5 standard deviations)
+        lin.weight[:, 11] *= 1e-3
+    want = _want(x, lin, ln)
+    assert bool(want.isfinite().all())
+    got = linear_rows_hip(x, lin, ln=ln).double()
+    assert bool(got.isfinite().all())
+    cols = torch.arange(N, device=device) == 7 if where == "weight" else torch.ones(N, dtype=torch.bool, device=device)
+    assert float(((got - want)[:, cols]).abs().max()) <= 1e-6 * float(want[:, cols].abs().max())
+    if where == "weight":
+        assert float((got - want)[:, ~cols].norm()) < 1e-6 * float(want[:, ~cols].norm())
+
+
+@pytest.mark.parametrize("side", [-1, 0, 1, 256])
+@torch.no_grad()
+def test_default_choice_near_its_line(device, monkeypatch, side):
+    """fc1-shaped layers on both sides of the line (four and a half tiled workgroups per compute unit; 544 and
+    545 rows on 256): the default call gives the bits of the kernel that the line says."""
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    line = 32 * (-(-9 * cus // 128) - 1)  # the most rows that stay with the tiled kernel: 64 column tiles
+    rows = line + side
     lin, ln = _layer(2048, torch.float32, device, rows)
     x = torch.randn(rows, K, device=device)
     want = F.gelu(_want(x, lin, ln))
-    assert float((linear_rows_hip(x, lin, ln=ln, gelu=True).double() - want).norm() / want.norm()) < 1e-6
+    out = {}
+    for kernel in ("block", "tiled", ""):
+        if kernel:
+            monkeypatch.setenv("PAGED_HIP_LINEAR_KERNEL", kernel)
+        else:
+            monkeypatch.delenv("PAGED_HIP_LINEAR_KERNEL", raising=False)
+        out[kernel] = linear_rows_hip(x, lin, ln=ln, gelu=True)
+        assert float((out[kernel].double() - want).norm() / want.norm()) < 1e-6
+    assert not torch.equal(out["block"], out["tiled"])
+    assert torch.equal(out[""], out["block" if side > 0 else "tiled"])
 
 
 @pytest.mark.parametrize("where", ["weight", "norm"])

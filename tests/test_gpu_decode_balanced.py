@@ -41,6 +41,8 @@ def test_same_as_unsplit(device, lens, H, Hd, io, kv):
     print(f"balanced decode {lens[:6]} H {H} Hd {Hd} {io} {kv}", flush=True)
     args, lists = _batch(device, lens, H, Hd, io, kv)
     dev = [t.to(device) for t in args]
+    # (the balanced launch is the one that runs)
+    assert _lib.load().pa_decode_workspace_size(len(lens), H, Hd, dev[3].shape[1], DECODE_BALANCED) > 0
     want = paged_attention_decode_hip(*dev, split_blocks=0).float()
     out = torch.full_like(dev[0], 9.0)
     got = paged_attention_decode_hip(*dev, split_blocks=DECODE_BALANCED, out=out).float()

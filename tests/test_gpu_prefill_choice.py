@@ -3,7 +3,7 @@ default call against the 16-row kernel, which serves all of them."""
 import pytest
 import torch
 
-from src.kernels.hip_paged_attention import paged_attention_prefill_hip
+from src.kernels.hip_paged_attention import PREFILL_BALANCED, paged_attention_prefill_hip, prefill_workspace_size
 
 pytestmark = pytest.mark.gpu
 
@@ -18,6 +18,8 @@ def test_balanced_calls_on_two_streams_and_in_graphs(device, monkeypatch):
         table = torch.randint(0, 600, (len(lens), 188), generator=g, device=device, dtype=torch.int32)
         cases.append((q, k, v, table, torch.tensor(lens, dtype=torch.int32, device=device),
                       torch.full((len(lens),), 200, dtype=torch.int32, device=device)))
+    for q, k, _, table, _, _ in cases:  # (the balanced launch is the one that runs)
+        assert prefill_workspace_size(*q.shape, table.shape[1], PREFILL_BALANCED, k.dtype) > 0
     want = [paged_attention_prefill_hip(*c).clone() for c in cases]
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     torch.cuda.synchronize()

@@ -3,7 +3,7 @@ ordinary values, and against the 16-row kernel (fp32 matrix instructions) where 
 import pytest
 import torch
 
-from src.kernels.hip_paged_attention import paged_attention_prefill_hip
+from src.kernels.hip_paged_attention import PREFILL_BALANCED, paged_attention_prefill_hip, prefill_workspace_size
 
 pytestmark = pytest.mark.gpu
 
@@ -23,6 +23,8 @@ def _run(case, device, monkeypatch, kernel, balance="off"):
     q, k, v, table, lens, cur = case
     monkeypatch.setenv("PAGED_HIP_PREFILL_KERNEL", kernel)
     monkeypatch.setenv("PAGED_HIP_PREFILL_BALANCE", balance)
+    B, H, T, Hd = q.shape  # (the launch under test is the one that runs)
+    assert (prefill_workspace_size(B, H, T, Hd, table.shape[1], PREFILL_BALANCED, k.dtype) > 0) == (balance == "force")
     return paged_attention_prefill_hip(q.to(device), k.to(device), v.to(device), table.to(device),
                                        torch.tensor(lens, dtype=torch.int32, device=device),
                                        torch.tensor(cur, dtype=torch.int32, device=device)).cpu()
@@ -70,20 +72,68 @@ def test_values_without_a_finite_split(device, monkeypatch, where, value, Hd, ba
         pool[table[1, 4], 3, 5, Hd - 2] = value   # its last keys
     got = _run(case, device, monkeypatch, "wide", balance)
     ref = _run(case, device, monkeypatch, "tile")
-    # A NaN row may come out as NaN or as 0 (no positive weight sum); all else agrees, to 1e-5 (float32
-    # sums of up to 150 keys in another order) of the row's largest value.
+    # to 1e-5 (float32 sums of up to 150 keys in another order) of the row's largest value
     bound = 1e-5 * ref.nan_to_num(0, 0, 0).abs().amax(-1, keepdim=True).clamp(min=1.0).expand_as(ref)
-    both = got.isfinite() & ref.isfinite()
-    assert bool(((got - ref).abs() <= bound)[both & (got != 0) & (ref != 0)].all())
-    clean = torch.ones_like(ref, dtype=torch.bool)  # rows that see no planted value
+    same = (got - ref).abs() <= bound
+    reached = torch.zeros_like(ref, dtype=torch.bool)  # outputs that a planted value reaches
     if where == "q":
-        clean[0, 1, 137] = clean[1, 2, 3] = False
-    else:
-        # (row 25 of request 0 sees keys 0-35; a masked key's weight is 0, and 0 * inf is NaN)
-        clean[0, 1, 25 if where == "k" else 0:] = clean[1, 3] = False
-    assert bool(both[clean].all())
-    if abs(value) < 1e30:  # (a larger value times a weight of up to 2^8 overflows)
-        assert bool(both.all())
+        reached[0, 1, 137] = reached[1, 2, 3] = True
+    elif where == "k":
+        reached[0, 1, 25:] = reached[1, 3] = True  # (row 25 of request 0 sees keys 0-35)
+    else:  # (its own column)
+        reached[0, 1, :, 7] = reached[1, 3, :, Hd - 2] = True
+    assert bool(ref[~reached].isfinite().all()) and bool(same[~reached].all())
+    if abs(value) < 1e30:
+        assert bool(ref.isfinite().all()) and bool(same.all())
+    elif where == "v":
+        sees = reached.clone()  # rows that see the key; to the others its weight is 0, and 0 * inf is NaN
+        sees[0, 1, :25] = sees[1, 3, :69] = False
+        if abs(value) < float("inf"):  # (the value times a weight of up to 2^8 may overflow on the way)
+            both = got.isfinite() & ref.isfinite()
+            assert bool(same[reached & both].all()) and bool(both[reached & ~sees].all())
+            one = sees & (got.isfinite() != ref.isfinite())
+            assert bool((torch.where(got.isfinite(), got, ref).abs() > 1e35)[one].all())
+        else:
+            assert torch.equal(got[sees].isnan(), ref[sees].isnan())
+            assert torch.equal(got[sees].nan_to_num(0, 1, -1), ref[sees].nan_to_num(0, 1, -1))
+            assert bool((same | got.isnan())[reached & ~sees & ref.isfinite()].all())
+    else:  # scores without a number: a NaN row, or 0 (no positive weight sum)
+        number = ref.isfinite() & (ref != 0)
+        assert bool(same[reached & number].all())
+        assert bool((~got.isfinite() | (got == 0))[reached & ~number].all())
+
+
+@pytest.mark.parametrize("balance", ["off", "force"])
+@pytest.mark.parametrize("Hd", [64, 128])
+@pytest.mark.parametrize("where", ["k", "v", "q"])
+@pytest.mark.parametrize("value", [3.4028234663852886e38, -3.4028234663852886e38, 3e38])
+def test_values_that_only_fp32_products_hold(device, monkeypatch, where, value, Hd, balance):
+    """Finite results from values whose parts are not finite: the products are formed again in fp32, or the
+    outputs would be NaN. The other operand is small enough for every product to be finite."""
+    assert torch.tensor(value * 2.0**24, dtype=torch.float64).bfloat16().isinf()  # (V's leading part)
+    lens, T, d = [150, 70], 140, 7
+    q, k, v, table, _, _ = case = _case(Hd, lens, T, 11)
+    at = table[0, 2], 1, 3      # key 35 of request 0, head 1
+    last = table[1, 4], 3, 5    # the last key of request 1, head 3
+    if where == "v":  # that key's score is far below the others', its weight about 1e-9
+        q.abs_()
+        k.abs_()
+        for x in (at, last):
+            k[x] *= -1
+            v[x][d] = value
+    else:  # scores of size 1: value * 1e-37 among the products
+        big, small = (k, q) if where == "k" else (q, k)
+        small[..., d] = 1e-37
+        for x in (at, last) if where == "k" else ((0, 1, 137), (1, 2, 3)):
+            big[x][d] = value
+        if where == "k":
+            assert torch.tensor(value).bfloat16().isinf() or abs(value) < 3.39e38
+    want = _f64(case)
+    assert bool(want.isfinite().all())
+    got = _run(case, device, monkeypatch, "wide", balance).double()
+    assert bool(got.isfinite().all())
+    # fp32 sums of values of N(0, 1), and the planted one's weight, whose exponent of about 30 is rounded to fp32
+    assert bool(((got - want).abs() <= 1e-5 + 1e-4 * want.abs()).all())
 
 
 @pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12])
