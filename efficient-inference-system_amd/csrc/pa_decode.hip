@@ -11,6 +11,7 @@
 // The next block's K and V are loaded into a second register set while the current one is used.
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "pa_attention.h"
 
@@ -556,15 +557,16 @@ void decode_balanced_kernel(const AttnArgs a) {
       else ub = mid - 1;
     }
   }
-  // The wavefronts' states as one: put(d, M, l, acc[d]).
-  auto combined = [&](auto&& put) {
+  // The states of N wavefronts from w0 on as one, by their threads (t from 0): put(d, M, l, acc[d]).
+  auto combined = [&](auto n, int w0, int t, auto&& put) {
+    constexpr int N = decltype(n)::value;
     float M = kNegBig;
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, sm_m[ww]);
-    for (int d = threadIdx.x; d < HD; d += NW * kWave) {
+    for (int ww = w0; ww < w0 + N; ++ww) M = fmaxf(M, sm_m[ww]);
+    for (int d = t; d < HD; d += N * kWave) {
       float lsum = 0.f, A = 0.f;
 #pragma unroll
-      for (int ww = 0; ww < NW; ++ww) {
+      for (int ww = w0; ww < w0 + N; ++ww) {
         const float f = fast_exp2(sm_m[ww] - M);
         lsum = fmaf(sm_l[ww], f, lsum);
         A = fmaf(sm_acc[ww][d], f, A);
@@ -572,8 +574,9 @@ void decode_balanced_kernel(const AttnArgs a) {
       put(d, M, lsum, A);
     }
   };
-  auto write = [&](int req) {
-    combined([&](int d, float, float lsum, float A) {
+  const std::integral_constant<int, NW> all;
+  auto write = [&](auto n, int w0, int t, int req) {
+    combined(n, w0, t, [&](int d, float, float lsum, float A) {
       IO* op = static_cast<IO*>(a.out) + (int64_t)req * a.o_sb + (int64_t)h * a.o_sh;
       Elem<IO>::store(op + d, lsum > 0.f ? A / lsum : 0.f);
     });
@@ -616,10 +619,10 @@ void decode_balanced_kernel(const AttnArgs a) {
     walk_blocks<KV, HD, NW>(a, pt, h, jb, je, n, ids0, w, lane, qv, sm_acc, sm_m, sm_l);
     __syncthreads();
     if (whole) {
-      write(b);
+      write(all, 0, threadIdx.x, b);
     } else {
       float* mine = record(gang, first);
-      combined([&](int d, float M, float lsum, float A) {
+      combined(all, 0, threadIdx.x, [&](int d, float M, float lsum, float A) {
         if (d == 0) {
           __hip_atomic_store(mine, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __hip_atomic_store(mine + 1, lsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -647,30 +650,32 @@ void decode_balanced_kernel(const AttnArgs a) {
     sm_last[w] = arrive_last(tickets + (int64_t)req * a.H + h, np, seen);
   }
   __syncthreads();
-  for (int c = 0; c < cuts; ++c) {
-    if (!__builtin_amdgcn_readfirstlane(sm_last[c])) continue;
-    const int req = c == 0 ? cut[0] : cut[1];
+  // Each is merged by half of the wavefronts: wavefront w of G folds records w, w + G, ... eight at a
+  // time, their words all in flight. (Whichever gang merges a request, the order of its sums is the same.)
+  static_assert(HD % kWave == 0 && NW % 2 == 0, "whole lanes, two halves");
+  constexpr int DL = HD / kWave, kDeep = 8, G = NW / 2;
+  const int half = w / G, w0 = half * G;
+  const bool mine = half < cuts && __builtin_amdgcn_readfirstlane(sm_last[half]);
+  const int req = half == 0 ? cut[0] : cut[1];
+  if (mine) {
     int g0;
     const int np = __builtin_amdgcn_readfirstlane(pieces(req, g0));
     g0 = __builtin_amdgcn_readfirstlane(g0);
     const int first = __builtin_amdgcn_readfirstlane(sS[req]);
-    // Wavefront w folds records w, w + NW, ... four at a time, their words all in flight.
-    static_assert(HD % kWave == 0, "whole lanes");
-    constexpr int DL = HD / kWave;
     float m = kNegBig, l = 0.f, acc[DL] = {};
-    for (int p = w; p < np; p += 4 * NW) {
-      float rm[4], rl[4], ra[4][DL];
+    for (int p = w - w0; p < np; p += kDeep * G) {
+      float rm[kDeep], rl[kDeep], ra[kDeep][DL];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const float* x = record(g0 + (p + t * NW < np ? p + t * NW : np - 1), first);
+      for (int t = 0; t < kDeep; ++t) {
+        const float* x = record(g0 + (p + t * G < np ? p + t * G : np - 1), first);
         rm[t] = rec_load<true>(x);
         rl[t] = rec_load<true>(x + 1);
 #pragma unroll
         for (int e = 0; e < DL; ++e) ra[t][e] = rec_load<true>(x + 2 + lane + e * kWave);
       }
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        if (p + t * NW >= np) break;
+      for (int t = 0; t < kDeep; ++t) {
+        if (p + t * G >= np) break;
         const float mn = fmaxf(m, rm[t]);
         const float fa = fast_exp2(m - mn), fr = fast_exp2(rm[t] - mn);
         l = l * fa + rl[t] * fr;
@@ -685,10 +690,10 @@ void decode_balanced_kernel(const AttnArgs a) {
       sm_m[w] = m;
       sm_l[w] = l;
     }
-    __syncthreads();
-    write(req);
-    __syncthreads();
   }
+  __syncthreads();
+  if (!mine) return;
+  write(std::integral_constant<int, G>(), w0, threadIdx.x - w0 * kWave, req);
 }
 
 // ---------------------------------------------------------------------------------------------
