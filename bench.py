@@ -564,6 +564,11 @@ def _prefill_metadata(device, lists, prev_lens, chunk_lens, T):
     return pt, s32, i32(chunk_lens), slots
 
 
+# Peak of the long-prompt kernels over fp32 KV: six bf16 partial products per fp32 product, on the bf16
+# matrix cores (the 16-row kernel's fp32 matrix instructions have 157.3).
+FP32_PARTS_PEAK = round(2500.0 / 6, 1)
+
+
 def _large_prefill(res, device, steps):
     import torch
 
@@ -577,7 +582,7 @@ def _large_prefill(res, device, steps):
         call = lambda: paged_attention_prefill_hip(b.q, b.k_pool, b.v_pool, b.page_table, b.seq_lens_t, b.cur_lens_t)
         ms = time_call(call, max(3, steps // 2))
         graph_ms = time_graph_call(call, calls=10 if tag == "bf16kv" else 4, replays=3)
-        peak = 157.3 if tag == "fp32" else 2500.0
+        peak = FP32_PARTS_PEAK if tag == "fp32" else 2500.0
         tfs = flops / (ms * 1e-3) / 1e12
         res[f"large_prefill_{tag}"] = {
             "workload": f"{b.batch} requests, {H} heads x {Hd}, context {b.extra['prev_lens']} + chunk 512 each, "
@@ -618,9 +623,9 @@ def _long_prompt_prefill(res, device, steps):
     # tile counts) is timed beside it.
     for kv_dtype, tag, peak, H, Hd, chunk, ctx, per_cu in (
             (torch.bfloat16, "bf16kv", 2500.0, 32, 128, 512, 8192, "two workgroups"),
-            (torch.float32, "fp32", 157.3, 32, 128, 512, 8192, "two workgroups"),
+            (torch.float32, "fp32", FP32_PARTS_PEAK, 32, 128, 512, 8192, "two workgroups"),
             (torch.bfloat16, "bf16kv_head_dim_64", 2500.0, 8, 64, 128, 32768, "one workgroup"),
-            (torch.float32, "fp32_head_dim_64", 157.3, 8, 64, 128, 32768, "one workgroup")):
+            (torch.float32, "fp32_head_dim_64", FP32_PARTS_PEAK, 8, 64, 128, 32768, "one workgroup")):
         b = workloads.large_prefill(seed=16, device=device, batch=1, heads=H, head_dim=Hd, chunk=chunk,
                                     ctx_lo=ctx, ctx_hi=ctx, kv_dtype=kv_dtype)
         flops = workloads.prefill_flops(b.extra["prev_lens"], b.cur_lens, H, Hd)

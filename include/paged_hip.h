@@ -135,24 +135,26 @@ int pa_decode_noalloc(const void* q, int64_t q_stride_b, int64_t q_stride_h,
  * Paged chunked-PREFILL attention (any query_len >= 1), causal over cached context plus the
  * in-chunk prefix. Replaces paged_attention_prefill_triton
  * (src/kernels/triton_paged_attention.py:220-258) behind paged_attention()
- * (src/kernels/paged_attention.py:44-51). fp32 KV uses fp32 MFMA (16x16x4); bf16 KV uses bf16
- * MFMA with fp32 accumulation (q and the softmax weights are rounded to bf16 for the products).
- * Work is one workgroup per (request, head, 16-row query tile); with split_blocks > 0 each tile's
- * KV blocks are also cut into ranges of split_blocks blocks, one workgroup each, whose partial
- * results a second kernel merges through a workspace of pa_prefill_workspace_size() bytes.
- * split_blocks == 0 means no split and no workspace. split_blocks < 0 (PA_PREFILL_BALANCED) asks
- * for the balanced launch where the library finds it faster: head_dim 128 or 64, num_heads a
- * multiple of 8, batch <= 255, at most one (request, head, 128-row tile) unit per two compute units
- * and at head_dim 128 at least 8192 unit-steps (units x ceil(max_pages / 2); fp32 KV: 4096 from one
- * unit per four compute units); at head_dim 64 at least 16384 unit-steps (steps of 64 keys for bf16
- * KV, 32 for fp32 KV) or 256 steps per unit (fp32 KV: at most one unit per 16 compute units), for
- * fp32 KV not where the 16-row kernel would run one to two workgroups per compute unit; i.e. few
- * tiles over long contexts. It runs a grid of one or two workgroups per compute unit, deals the tiles' KV steps out
- * evenly among them and merges a tile cut between workgroups in the same launch (the one that
+ * (src/kernels/paged_attention.py:44-51). bf16 KV uses bf16 MFMA with fp32 accumulation (q and the
+ * softmax weights are rounded to bf16 for the products). fp32 KV keeps fp32 products: the 16-row kernel
+ * on fp32 MFMA (16x16x4), the 128-row kernels as the six leading partial products of operands in three
+ * bf16 parts each, on bf16 MFMA with fp32 accumulation; tiles that meet a K, V or scaled q of 2^60 or more
+ * (infinities among them) form theirs again on fp32 MFMA.
+ * An unsplit call takes the kernel of the least estimated time for its sizes and the page table's width:
+ * 16-row tiles, 32-row split-step tiles (bf16 KV, head_dim 64), 128-row tiles or the balanced launch. With
+ * split_blocks > 0 each 16-row tile's KV blocks are cut into ranges of split_blocks blocks, one
+ * workgroup each, whose partial results a second kernel merges through a workspace of
+ * pa_prefill_workspace_size() bytes. split_blocks == 0 means no split, no balanced launch and no
+ * workspace. split_blocks < 0 (PA_PREFILL_BALANCED) allows the balanced launch: head_dim 128 or 64,
+ * num_heads a multiple of 8, batch <= 255, at most two (request, head, 128-row tile) units per
+ * compute unit, and at head_dim 64 with at most half a unit per compute unit only page tables of 192
+ * blocks and more. It runs a grid of one or two workgroups per compute unit, deals the tiles' KV steps
+ * out evenly among them and merges a tile cut between workgroups in the same launch (the one that
  * finishes it last). Other calls run as with 0. The environment variable
  * PAGED_HIP_PREFILL_BALANCE=force takes it wherever it can run (as many workgroups per compute
- * unit as fit on larger grids), =off never. Every prefill workspace starts with PA_PREFILL_COUNTER_BYTES of
- * arrival counters that must be zero before its first use; every call leaves them zero. Calls that
+ * unit as fit on larger grids), =off never. Every prefill workspace starts with
+ * PA_PREFILL_COUNTER_BYTES of arrival counters that must be zero before its first use; every call
+ * leaves them zero. Calls that
  * share a workspace must not run concurrently (e.g. on different streams).
  */
 int pa_prefill(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
