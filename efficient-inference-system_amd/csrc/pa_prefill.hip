@@ -659,6 +659,13 @@ static bool prefill_fast_shape(int32_t head_dim, int32_t block_size) {
 // per compute unit over long contexts (fp32, 8 x 32 x 128, 128 rows over 6k: wide 600, balanced 392;
 // 8 x 8 x 64, 512 rows 358 / 190, bf16 94 / 55) and few rows over long contexts at head_dim 64
 // (bf16, 4 x 8 heads, 64 rows over 6k: 16-row 29, split-step 20; fp32, 1 x 8: 16-row 53, balanced 37).
+// The rule sees the table's width, not the lengths in it. Over tables 4 to 500 times as wide as their
+// contexts it stays ahead of the unit counts in the mean (0.81-0.97 of their times; fp32 at head_dim 64
+// 1.03), but single calls lose: the balanced launch takes 12-30 us over contexts of 60-256 tokens, the
+// 16-row kernel 5-13 (fp32, 4 x 8 x 64, 128 rows over 256 tokens, 512-page table: 6.5 -> 17.9). Past the
+// fitted contexts, over 9-12k tokens, 1-4 requests of 32 heads x 128 with up to 64 rows take the 16-row
+// kernel where the balanced launch is up to 29% faster (bf16, 2 x 32, 16 rows: 81 / 63); a line that
+// gave it those would give it the short contexts under such tables too, at three times the time.
 // The lines that the estimates do not draw:
 //   - balanced up to two tiles per compute unit (beyond, the tiles fill the grid's end by themselves:
 //     fp32, 32 x 8 x 64, 512 rows over 1.5k 231 wide, 274 balanced) and, at head_dim 64 with at most
